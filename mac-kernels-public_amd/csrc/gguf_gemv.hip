@@ -40,6 +40,7 @@ constexpr int GV_THREADS = 256;
 constexpr int GV_MAX_K = 8192;
 
 typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32a2 __attribute__((aligned(2)));
 
 __device__ __forceinline__ f16x2 h2(uint32_t u) { return __builtin_bit_cast(f16x2, u); }
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
@@ -326,7 +327,9 @@ template <> struct GV<gguf::Q6_K> {
         r[26] = sc[0];
         r[27] = sc[1];
         r[28] = sc[sh ? 2 : 1];
-        r[29] = *reinterpret_cast<const uint16_t*>(b + 208);
+        // d in the upper half of the block's last dword (2-byte aligned): a 16-bit load held across a
+        // loop would be masked, and so waited for, at the loop's end
+        r[29] = *reinterpret_cast<const u32a2*>(b + 206);
         r[30] = (uint32_t)sh;
     }
     // alignbyte with shift 0 returns its low operand: the same code serves both alignments
@@ -338,7 +341,7 @@ template <> struct GV<gguf::Q6_K> {
         for (int i = 17; i < 25; ++i) q[i] = __builtin_amdgcn_alignbyte(r[i + 1], r[i], sh);
         q[26] = __builtin_amdgcn_alignbyte(r[27], r[26], sh);
         q[27] = __builtin_amdgcn_alignbyte(r[28], r[27], sh);
-        q[29] = r[29];
+        q[29] = r[29] >> 16;
     }
     // ql dword j: low nibbles -> values 4j..4j+3, high nibbles -> 64 + 4j..; natural pairing (x0,x2),(x1,x3)
     __device__ static void prep_x(const uint32_t* xn, uint32_t* xp, float* xs) {
@@ -509,7 +512,7 @@ hipError_t launch(const GgufGemvArgs& a, hipStream_t st) {
     if (blocks < 1) blocks = 1;
     dim3 grid((unsigned)blocks), block(GV_THREADS);
 #define QLIN_GV(L)                                                                                      \
-    hipLaunchKernelGGL((gguf_gemv_kernel<T, L>), grid, block, 0, st, a.x, a.xexp, a.w, a.row_bytes, a.N, a.K, a.bias, \
+    hipLaunchKernelGGL((gguf_gemv_kernel<T, L>), grid, block, 0, st, (const f16*)a.x, a.xexp, a.w, a.row_bytes, a.N, a.K, a.bias, \
                        a.bias_dtype, a.y, a.y_dtype)
     switch (lpr) {
         case 16: QLIN_GV(16); break;
@@ -518,6 +521,380 @@ hipError_t launch(const GgufGemvArgs& a, hipStream_t st) {
         default: return hipErrorInvalidValue;
     }
 #undef QLIN_GV
+    return hipGetLastError();
+}
+
+
+// --------------------------------------------------------------------------------------------
+// Rows of any length (and bf16 / fp32 rows of every length): LPR lanes walk a row's chunks c = l,
+// l + LPR, ..., with the loads of two chunks in flight per lane.  The operand order of the activations
+// is made once per workgroup, in LDS, instead of once per lane in registers (a wave's chunks change),
+// and bf16 / fp32 rows are normalized there, where the prologue was a launch of its own.  Bound by
+// the weight stream, the decode's VALU (Q4_K: 5 operations per two weights) and, at a few MB, by the
+// latency of the first bytes.  In a HIP graph over cold weights, us against the kernels that these
+// rows took before (the small-M one, or the prologue and the kernel below): Q4_K K5120 N13824 bf16
+// 13.7 against 30.8 (2.9 TB/s), Q6_K K13824 N5120 bf16 22.0 against 45.2, IQ4_XS K14336 N4096 bf16
+// 12.8 against 23.4, Q8_0 K11264 N4096 bf16 11.9 against 20.8, Q4_K K = N = 4096 bf16 5.4 against
+// 7.5.  fp16 rows keep the kernel below at its K (Q4_K 5.0, Q6_K 5.6, Q8_0 5.6 us there).
+//
+// LDS operand: 16-byte unit i (8 values) of chunk c at i * C + c, so that the lanes of a row read
+// consecutive units.  Byte codes: each 8 values as the pairs (0,2) (1,3) (4,6) (5,7).  Table
+// formats: unit 4 b + q of a chunk holds the pairs (x_j, x_j+16), j = 4 q .. + 3, of its block b.
+// Codes become exact fp16 integers (1024 + q less 1024 in one packed add), so no offset term cancels
+// against the sums; the K-quants' minima take sums of 32 activations, at g * C + c.
+// --------------------------------------------------------------------------------------------
+template <int OFF>
+__device__ __forceinline__ uint32_t less(uint32_t pair) {  // an fp16 pair minus (OFF, OFF)
+    return __builtin_bit_cast(uint32_t, h2(pair) - f16x2{(f16)OFF, (f16)OFF});
+}
+template <int T>
+struct GVRow {  // Q4_K, Q5_K
+    template <typename XU, typename XS>
+    __device__ static float dot(const uint32_t* r, int c, XU&& xu, XS&& xs, const uint32_t*) {
+        const int h = c & 1;
+        const float d = f16_bits_to_f32((uint16_t)(r[0] & 0xFFFFu)), dmin = f16_bits_to_f32((uint16_t)(r[0] >> 16));
+        const uint32_t s0 = r[1], s1 = r[2], s2 = r[3];
+        constexpr int QB = (T == gguf::Q4_K) ? 4 : 12;
+        float S[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < 2; ++p)  // sub-blocks 2p (low nibbles), 2p + 1 (high)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32x4 xl = xu(8 * p + q), xh = xu(8 * p + 4 + q);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t w = r[QB + 8 * p + 2 * q + e];
+                    const uint32_t l0 = e ? xl.z : xl.x, l1 = e ? xl.w : xl.y, h0 = e ? xh.z : xh.x, h1 = e ? xh.w : xh.y;
+                    if constexpr (T == gguf::Q5_K) {
+                        const uint32_t qh = r[4 + 2 * q + e];
+                        const int sb = 4 * h + 2 * p;
+                        const uint32_t lo = (w & 0x0F0F0F0Fu) | (((qh >> sb) & 0x01010101u) << 4);
+                        const uint32_t hi = ((w >> 4) & 0x0F0F0F0Fu) | (((qh >> (sb + 1)) & 0x01010101u) << 4);
+                        S[2 * p] = dot2(less<1024>(byte_pair(lo)), l0, S[2 * p]);
+                        S[2 * p] = dot2(less<1024>(byte_pair_hi(lo)), l1, S[2 * p]);
+                        S[2 * p + 1] = dot2(less<1024>(byte_pair(hi)), h0, S[2 * p + 1]);
+                        S[2 * p + 1] = dot2(less<1024>(byte_pair_hi(hi)), h1, S[2 * p + 1]);
+                    } else {  // high nibbles as 16 q (no shift)
+                        S[2 * p] = dot2(less<1024>(nib_pair(w)), l0, S[2 * p]);
+                        S[2 * p] = dot2(less<1024>(nib_pair(w >> 8)), l1, S[2 * p]);
+                        S[2 * p + 1] = dot2(less<1024>(nib16_pair(w)), h0, S[2 * p + 1]);
+                        S[2 * p + 1] = dot2(less<1024>(nib16_pair(w >> 8)), h1, S[2 * p + 1]);
+                    }
+                }
+            }
+        // the chunk's four 6-bit scales and minima as bytes, for both halves without a branch
+        const uint32_t hm = 0u - (uint32_t)h;
+        const uint32_t sc = (((s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u)) & hm) | (s0 & 0x3F3F3F3Fu & ~hm);
+        const uint32_t mn = ((((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u)) & hm) | (s1 & 0x3F3F3F3Fu & ~hm);
+        float acc = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float a = d * (float)((sc >> (8 * g)) & 0xFFu), b = dmin * (float)((mn >> (8 * g)) & 0xFFu);
+            acc += (T == gguf::Q4_K && (g & 1) ? 0.0625f * a : a) * S[g] - b * xs(g);
+        }
+        return acc;
+    }
+};
+template <>
+struct GVRow<gguf::Q6_K> {
+    template <typename XU, typename XS>
+    __device__ static float dot(const uint32_t* raw, int, XU&& xu, XS&&, const uint32_t*) {
+        uint32_t r[30];
+        GV<gguf::Q6_K>::realign(raw, r);
+        const float d = f16_bits_to_f32((uint16_t)(r[29] & 0xFFFFu));
+        float S[8];
+#pragma unroll
+        for (int g = 0; g < 8; ++g) S[g] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {  // values 8q .. + 7 (low nibbles), 64 + 8q .. + 7 (high)
+            const u32x4 xl = xu(q), xh = xu(8 + q);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int j = 2 * q + e, sl = 2 * (j / 8), glo = j / 4, ghi = 4 + j / 4;
+                const uint32_t ql = r[j], qh = r[17 + (j % 8)];
+                const uint32_t lo = (ql & 0x0F0F0F0Fu) | (((qh >> sl) & 0x03030303u) << 4);
+                const uint32_t hi = ((ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (sl + 4)) & 0x03030303u) << 4);
+                S[glo] = dot2(less<1056>(byte_pair(lo)), e ? xl.z : xl.x, S[glo]);
+                S[glo] = dot2(less<1056>(byte_pair_hi(lo)), e ? xl.w : xl.y, S[glo]);
+                S[ghi] = dot2(less<1056>(byte_pair(hi)), e ? xh.z : xh.x, S[ghi]);
+                S[ghi] = dot2(less<1056>(byte_pair_hi(hi)), e ? xh.w : xh.y, S[ghi]);
+            }
+        }
+        float acc = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const int sc = (int)(int8_t)(r[26 + g / 4] >> (8 * (g % 4)));
+            acc += (d * (float)sc) * S[g];
+        }
+        return acc;
+    }
+};
+template <>
+struct GVRow<gguf::Q8_0> {
+    template <typename XU, typename XS>
+    __device__ static float dot(const uint32_t* r, int, XU&& xu, XS&&, const uint32_t*) {
+        float acc = 0.0f;
+        static_for<2>([&](auto B) {
+            constexpr int b = decltype(B)::value, o = 34 * b;
+            float S = 0.0f;
+            static_for<4>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                const u32x4 xv = xu(4 * b + q);
+                const uint32_t w0 = dw_at<o + 2 + 8 * q>(r) ^ 0x80808080u, w1 = dw_at<o + 6 + 8 * q>(r) ^ 0x80808080u;
+                S = dot2(less<1152>(byte_pair(w0)), xv.x, S);
+                S = dot2(less<1152>(byte_pair_hi(w0)), xv.y, S);
+                S = dot2(less<1152>(byte_pair(w1)), xv.z, S);
+                S = dot2(less<1152>(byte_pair_hi(w1)), xv.w, S);
+            });
+            acc += half_at<o>(r) * S;
+        });
+        return acc;
+    }
+};
+// four bytes of codes against one unit: a table entry is the fp16 pair of a byte's two values
+__device__ __forceinline__ float tab_dot(uint32_t w, const u32x4& xv, const uint32_t* tab, float S) {
+    S = dot2(tab[w & 0xFFu], xv.x, S);
+    S = dot2(tab[(w >> 8) & 0xFFu], xv.y, S);
+    S = dot2(tab[(w >> 16) & 0xFFu], xv.z, S);
+    return dot2(tab[w >> 24], xv.w, S);
+}
+template <int T>
+struct GVRowTab32 {
+    template <typename XU, typename XS>
+    __device__ static float dot(const uint32_t* r, int, XU&& xu, XS&&, const uint32_t* tab) {
+        float acc = 0.0f;
+        static_for<4>([&](auto B) {
+            constexpr int b = decltype(B)::value, o = 18 * b;
+            float S = 0.0f;
+            static_for<4>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                S = tab_dot(dw_at<o + 2 + 4 * q>(r), xu(4 * b + q), tab, S);
+            });
+            acc += half_at<o>(r) * S;
+        });
+        return acc;
+    }
+};
+template <> struct GVRow<gguf::Q4_0> : GVRowTab32<gguf::Q4_0> {};
+template <> struct GVRow<gguf::IQ4_NL> : GVRowTab32<gguf::IQ4_NL> {};
+template <>
+struct GVRow<gguf::IQ4_XS> {
+    template <typename XU, typename XS>
+    __device__ static float dot(const uint32_t* r, int c, XU&& xu, XS&&, const uint32_t* tab) {
+        const int h = c & 1;
+        const float d = f16_bits_to_f32((uint16_t)(r[0] & 0xFFFFu));
+        const uint32_t sh = r[0] >> 16, sl = r[1];
+        float acc = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int s = 4 * h + g;
+            const int ls = ((sl >> (8 * (s >> 1) + 4 * (s & 1))) & 0xF) | (int)(((sh >> (2 * s)) & 3u) << 4);
+            float S = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) S = tab_dot(r[2 + 4 * g + q], xu(4 * g + q), tab, S);
+            acc += (d * (float)(ls - 32)) * S;
+        }
+        return acc;
+    }
+};
+
+constexpr int GVR_THREADS = 256;
+constexpr int GVR_MAX_K = 16384;  // 32 KiB of operand in LDS
+
+// 8 raw activations as loaded (held until the weight loads are out)
+template <typename TX> struct RawUnit {
+    u32x4 v[sizeof(TX) / 2];
+    __device__ void load(const TX* p) {
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(TX) / 2; ++i) v[i] = reinterpret_cast<const u32x4*>(p)[i];
+    }
+    __device__ float get(int e) const {
+        if constexpr (sizeof(TX) == 4) return __uint_as_float(v[e / 4][e % 4]);
+        else return bf16_bits_to_f32((uint16_t)(v[0][e / 2] >> (16 * (e % 2))));
+    }
+};
+
+template <int T, int LPR, typename TX>
+__global__ __launch_bounds__(GVR_THREADS) void gguf_gemv_rows_kernel(const TX* x, const int32_t* xexp, const uint8_t* w,
+                                                            int64_t row_bytes, int N, int K, const void* bias,
+                                                            int bias_dt, void* y, int y_dt) {
+    using F = GV<T>;
+    constexpr bool RAW = !std::is_same<TX, f16>::value;  // fp16 rows are used as they are
+    constexpr bool TAB = F::LUT;
+    constexpr int NT = GVR_THREADS, NW = NT / 64, NX = GVR_MAX_K / 8 / NT;
+    constexpr int VC = F::VC, RPW = 64 / LPR;
+    constexpr bool MIN = T == gguf::Q4_K || T == gguf::Q5_K;  // block minima: sums of x per 32 values
+    __shared__ __attribute__((aligned(16))) u32x4 xop[GVR_MAX_K / 8];
+    __shared__ float xsum[MIN ? GVR_MAX_K / 32 : 1];
+    __shared__ uint32_t tab_all[TAB ? NW : 1][TAB ? 256 : 1];
+    __shared__ float red[NW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane % LPR, KU = K / 8, C = K / VC, IT = (C + LPR - 1) / LPR;
+    const int nwaves = gridDim.x * NW, groups = (N + RPW - 1) / RPW;
+    int g = blockIdx.x * NW + wave;                      // this wave's row group; then g + nwaves, ...
+    auto row = [&](int gg) { return min(gg * RPW + lane / LPR, N - 1); };
+
+    // the activations' loads first (units past the row re-read its last), then two chunks' weights
+    RawUnit<TX> xv[NX];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) xv[j].load(x + 8 * min(tid + NT * j, KU - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t r0[F::LD], r1[F::LD];
+    // Loads run two chunks ahead of the sums, across the end of a row group into the next one; they
+    // are unconditional (past the last chunk they re-read it), so that the compiler's wait for the
+    // older of the two does not cover the newer.
+    int fg = g, fit = 0;
+    const uint8_t* frow = w + (int64_t)row(g) * row_bytes;
+    auto fetch = [&](uint32_t* r) {
+        F::load(frow, min(l + LPR * fit, C - 1), r);
+        if (++fit == IT) {
+            if (fg + nwaves < groups) {
+                fg += nwaves;
+                fit = 0;
+                frow = w + (int64_t)row(fg) * row_bytes;
+            } else {
+                fit = IT - 1;
+            }
+        }
+    };
+    fetch(r0);
+    fetch(r1);
+    const int xe = xexp ? xexp[0] : 0;
+    uint32_t bv = bias ? load_bits_rt(bias, bias_dt, row(g)) : 0u;
+    __builtin_amdgcn_sched_barrier(0);
+
+    int E = xe;
+    if constexpr (RAW) {  // the prologue's normalization: fp16(x 2^-E), E the exponent of max |x|
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NX; ++j)
+            if (NT * j < KU) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(xv[j].get(e)));
+            }
+        amax = wave_max(amax);
+        if (lane == 0) red[wave] = amax;
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < NW; ++i) amax = fmaxf(amax, red[i]);
+        E = frexp_exp(amax);
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+        if (NT * j >= KU) break;
+        const int u = tid + NT * j;
+        uint32_t h[4];  // the unit's fp16 pairs in natural order
+        if constexpr (RAW) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const f16 a = (f16)__builtin_ldexpf(xv[j].get(2 * e), -E), b = (f16)__builtin_ldexpf(xv[j].get(2 * e + 1), -E);
+                h[e] = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = xv[j].v[0][e];
+        }
+        constexpr int UC = VC / 8;
+        const int c = u / UC, i = u % UC;
+        u32x4 o;
+        if constexpr (TAB) {
+            // lanes t and t ^ 2 hold the same 8 places of a block's two halves: the lower makes its
+            // first four pairs (x_j, x_j+16), the upper its last four
+            const bool up = tid & 2;
+            const uint32_t s0 = up ? h[0] : h[2], s1 = up ? h[1] : h[3];
+            const uint32_t t0 = __shfl_xor((int)s0, 2, 64), t1 = __shfl_xor((int)s1, 2, 64);
+            const uint32_t a0 = up ? t0 : h[0], a1 = up ? t1 : h[1], b0 = up ? h[2] : t0, b1 = up ? h[3] : t1;
+            o = u32x4{lo_lo(a0, b0), hi_hi(a0, b0), lo_lo(a1, b1), hi_hi(a1, b1)};
+            const int k4 = i % 4;  // units 0, 2, 1, 3 of a block make pairs 0 .. 3, 4 .. 7, 8 .. 11, 12 .. 15
+            if (u < KU) xop[(i - k4 + 2 * (k4 & 1) + (k4 >> 1)) * C + c] = o;
+        } else {
+            o = u32x4{lo_lo(h[0], h[1]), hi_hi(h[0], h[1]), lo_lo(h[2], h[3]), hi_hi(h[2], h[3])};
+            if (u < KU) xop[i * C + c] = o;
+            if constexpr (MIN) {
+                float s = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s = pair_sum(h[e], s);
+                s += lane_xor<1>(s);
+                s += lane_xor<2>(s);
+                if (u < KU && u % 4 == 0) xsum[(i / 4) * C + c] = s;
+            }
+        }
+    }
+    uint32_t* tab = tab_all[TAB ? wave : 0];
+    if constexpr (TAB) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tab[lane + 64 * i] = table_entry<T>(lane + 64 * i);
+    }
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);  // nothing that needs a weight value moves above this point
+
+    float acc = 0.0f;
+    int it = 0;
+    auto step = [&](uint32_t* r) {
+        const int cc = l + LPR * it, c = min(cc, C - 1);
+        const float v = GVRow<T>::dot(r, c, [&](int i) { return xop[i * C + c]; }, [&](int i) { return xsum[i * C + c]; }, tab);
+        acc += cc < C ? v : 0.0f;
+        // the refill goes into the registers just used: issued before the sum is done (the empty asm
+        // pins it) it would need others, and a copy, a wait for the load, at the end of the loop
+        asm volatile("" : "+v"(acc));
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(r);
+        __builtin_amdgcn_sched_barrier(0);
+        if (++it == IT) {
+#pragma unroll
+            for (int m = 1; m < LPR; m <<= 1) acc += __shfl_xor(acc, m, 64);
+            const int n = g * RPW + lane / LPR;
+            if (l == 0 && n < N) store_rt(y, y_dt, n, __builtin_ldexpf(acc, E) + bits_to_f32_rt(bv, bias_dt));
+            g += nwaves;
+            if (bias) bv = load_bits_rt(bias, bias_dt, row(g));  // past the last group: row N - 1, not used
+            acc = 0.0f;
+            it = 0;
+        }
+    };
+    const int steps = g < groups ? ((groups - g + nwaves - 1) / nwaves) * IT : 0;
+    for (int s = 1; s < steps; s += 2) {
+        step(r0);
+        step(r1);
+    }
+    if (steps & 1) step(r0);
+}
+
+// Lanes per row L and row groups per wave G.  The fastest grids measured have at most 1024 waves (a
+// workgroup of 4 per CU: with more than one workgroup on some CUs they wait for those, and each
+// redoes the operand); of those, the shortest wave: G row groups of IT chunks and one reduction
+// each.  us for each L at its best G, the one taken first (before the codes were made exact): Q4_K
+// K5120 N13824 L8 11.2, L16 12.3, L32 14.7; Q6_K K13824 N5120 L8 23.0, L16 22.1, L32 22.1; Q8_0 K11264
+// N4096 L16 11.9, L64 11.2; Q4_K K3072 N3072 L16 4.6, L32 5.0, L8 5.4; Q4_K K8192 N1024 L64 4.4, L32 5.0.
+inline int gemv_rows_lanes(int N, int C, int& G) {
+    int best = 0, L = 8;
+    for (int l : {8, 16, 32, 64}) {
+        const int64_t waves = ((int64_t)N * l + 63) / 64;
+        const int g = (int)((waves + 1023) / 1024), cost = g * ((C + l - 1) / l + 1);
+        if (!best || cost < best) {
+            best = cost;
+            L = l;
+            G = g;
+        }
+    }
+    return L;
+}
+
+template <int T, typename TX>
+hipError_t launch_rows(const GgufGemvArgs& a, hipStream_t st) {
+    int G = 1;
+    const int L = gemv_rows_lanes(a.N, a.K / GV<T>::VC, G);
+    const int64_t rows = (int64_t)GVR_THREADS / L * G;
+    const dim3 grid((unsigned)((a.N + rows - 1) / rows)), block(GVR_THREADS);
+#define QLIN_GVR(LV)                                                                                                   \
+    hipLaunchKernelGGL((gguf_gemv_rows_kernel<T, LV, TX>), grid, block, 0, st, (const TX*)a.x, a.xexp, a.w, a.row_bytes, \
+                       a.N, a.K, a.bias, a.bias_dtype, a.y, a.y_dtype)
+    switch (L) {
+        case 8: QLIN_GVR(8); break;
+        case 16: QLIN_GVR(16); break;
+        case 32: QLIN_GVR(32); break;
+        default: QLIN_GVR(64); break;
+    }
+#undef QLIN_GVR
     return hipGetLastError();
 }
 
@@ -536,6 +913,25 @@ bool dispatch_gemv(int t, Fn&& f) {
 }
 
 }  // namespace
+
+bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void* w, const void* x) {
+    // Q6_K rows of an odd number of blocks start 2 bytes off a dword, which its loads realign
+    if (K > GVR_MAX_K || (uintptr_t)w % 4 || (uintptr_t)x % 16 || row_bytes % (type == gguf::Q6_K ? 2 : 4)) return false;
+    bool ok = false;
+    dispatch_gemv(type, [&]<int T>() { ok = K % GV<T>::VC == 0; });
+    return ok;
+}
+
+hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st) {
+    if (a.y_dtype != DT_F32 && a.y_dtype != DT_F16 && a.y_dtype != DT_BF16) return hipErrorInvalidValue;
+    hipError_t err = hipErrorInvalidValue;
+    dispatch_gemv(a.type, [&]<int T>() {
+        if (a.x_dtype == DT_F16) err = launch_rows<T, f16>(a, st);
+        else if (a.x_dtype == DT_BF16) err = launch_rows<T, bf16_t>(a, st);
+        else if (a.x_dtype == DT_F32) err = launch_rows<T, float>(a, st);
+    });
+    return err;
+}
 
 bool gguf_gemv_supported(int type, int64_t M, int64_t K, int64_t row_bytes, const void* w, const void* x) {
     if (M != 1 || K > GV_MAX_K || (uintptr_t)w % 4 || (uintptr_t)x % 16 || row_bytes % 4) return false;

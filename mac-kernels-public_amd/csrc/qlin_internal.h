@@ -168,8 +168,9 @@ hipError_t run_int8_gemv(const Int8GemvArgs& a, hipStream_t st);
 
 struct GgufGemvArgs {
     int type = 0;
-    const f16* x = nullptr;          // one fp16 activation row (16-byte aligned)
-    const int32_t* xexp = nullptr;   // its exponent to restore (nullptr = 0)
+    const void* x = nullptr;         // one activation row (16-byte aligned)
+    int x_dtype = DT_F16;            // f16: used as it is; bf16 / f32 (run_gguf_gemv_rows): normalized in the kernel
+    const int32_t* xexp = nullptr;   // an fp16 row's exponent to restore (nullptr = 0)
     const uint8_t* w = nullptr;
     int64_t row_bytes = 0;
     int N = 0, K = 0;
@@ -180,6 +181,9 @@ struct GgufGemvArgs {
 };
 bool gguf_gemv_supported(int type, int64_t M, int64_t K, int64_t row_bytes, const void* w, const void* x);
 hipError_t run_gguf_gemv(const GgufGemvArgs& a, hipStream_t st);
+// The GEMV over rows of any whole number of chunks (64 values for Q8_0, else 128) up to 16384.
+bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void* w, const void* x);
+hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st);
 
 // ---- weight-only fp16 MFMA tile GEMM (gemm_f16.hip) ----
 enum { WO_INT8 = 0, WO_GGUF = 1, WO_F16 = 2 };  // WO_F16: fp16 weights w[n] 2^-e[n] (a decoded GGUF tensor)
