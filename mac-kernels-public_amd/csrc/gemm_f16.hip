@@ -15,6 +15,7 @@
 #include "qlin_internal.h"
 #include "lora_frag.h"
 #include "gguf_exact.h"
+#include "gemm_pp.h"
 
 namespace qlin {
 namespace {
@@ -556,42 +557,24 @@ constexpr int wo_dma_lora_rank(int du) {
     return du == DT_F32 ? lora_max_rank<DT_F32, 256, 256>(lds) : lora_max_rank<DT_BF16, 256, 256>(lds);
 }
 
-template <int BMT, int STAGES, int LDU = -1>
+// PP: the main loop of gemm_pp.h instead (256 x 256 tiles, K a multiple of 128).
+template <int BMT, int STAGES, int LDU = -1, bool PP = false>
 __global__ __launch_bounds__(512) void gemm_wo_dma_kernel(GemmF16Args a) {
     constexpr int NT = 512, BNT = 256, KT = 64;
+    static_assert(!PP || BMT == 256, "256 x 256 tiles");
     // waves 2 (M) x 4 (N): each converted weight fragment feeds TI = 4 activation sub-tiles
     constexpr int WM = BMT / 2, WN = BNT / 4, TI = WM / 32, TJ = WN / 32;
     constexpr int ASZ = BMT * KT * 2, BSZ = BNT * KT;   // bytes per stage
     constexpr int NA = ASZ / 16 / NT, NB = BSZ / 16 / NT;
     static_assert(TI >= 1 && NA * 16 * NT == ASZ && NB * 16 * NT == BSZ, "tile shape");
     __shared__ __attribute__((aligned(16))) uint8_t smem[STAGES * (ASZ + BSZ)];
+    static_assert(!PP || PingPongW8::LDS <= (int)sizeof(smem), "operand buffers");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1, r32 = lane & 31, h = lane >> 5;
+    const int wm = PP ? wave >> 2 : wave & 1, wn = PP ? wave & 3 : wave >> 1, r32 = lane & 31, h = lane >> 5;
     int mt, nt;
     xcd_tile_f16(blockIdx.x, (int)gridDim.x, (int)((a.M + BMT - 1) / BMT), (int)((a.N + BNT - 1) / BNT), mt, nt);
     const int64_t n0 = (int64_t)nt * BNT, m0 = (int64_t)mt * BMT;
     const int ktiles = (int)(a.K / KT);
-
-    // DMA instruction i of wave w fills physical chunk u = NT i + 64 w + lane of a stage: activation
-    // row u / 8, weight row u / 4.  The logical chunk it holds is the same for every i.
-    const int ca = (lane % 8) ^ ((4 * wave + lane / 16) % 8);
-    const int cb = (lane % 4) ^ (lane / 16);
-    const f16* asrc[NA];
-    const int8_t* bsrc[NB];
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-        asrc[i] = a.x + min(m0 + (NT * i + 64 * wave + lane) / 8, a.M - 1) * a.ldx + 8 * ca;
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-        bsrc[i] = (const int8_t*)a.w + min(n0 + (NT * i + 64 * wave + lane) / 4, a.N - 1) * a.ldw + 16 * cb;
-    auto dma = [&](int kt, int buf) {
-        const int k0 = min(kt, ktiles - 1) * KT;  // past the end: re-reads the last tile
-        uint8_t* st = smem + buf * (ASZ + BSZ);
-#pragma unroll
-        for (int i = 0; i < NA; ++i) lds_dma16(asrc[i] + k0, st + 16 * (NT * i + 64 * wave));
-#pragma unroll
-        for (int i = 0; i < NB; ++i) lds_dma16(bsrc[i] + k0, st + ASZ + 16 * (NT * i + 64 * wave));
-    };
 
     f32x16 acc[TI][TJ];
 #pragma unroll
@@ -600,63 +583,89 @@ __global__ __launch_bounds__(512) void gemm_wo_dma_kernel(GemmF16Args a) {
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    // this lane's rows: activation rows wm WM + 32 i + r32 (swizzle (row / 2) % 8 = (r32 / 2) % 8
-    // since WM and 32 are multiples of 16), weight rows wn WN + 32 j + r32 (swizzle (r32 / 4) % 4)
-    const int swa = (r32 / 2) % 8, swb = (r32 / 4) % 4;
-    auto mfmas = [&](int buf) {
-        const uint8_t* as = smem + buf * (ASZ + BSZ) + (wm * WM + r32) * (KT * 2);
-        const uint8_t* bs = smem + buf * (ASZ + BSZ) + ASZ + (wn * WN + r32) * KT;
+    if constexpr (PP) {
+        PingPongW8::run(smem, (const uint8_t*)(a.x + m0 * a.ldx), a.ldx * 2, (int)min<int64_t>(BMT, a.M - m0),
+                        (const uint8_t*)a.w + n0 * a.ldw, a.ldw, (int)min<int64_t>(BNT, a.N - n0), ktiles, tid, acc);
+    } else {
+        // DMA instruction i of wave w fills physical chunk u = NT i + 64 w + lane of a stage: activation
+        // row u / 8, weight row u / 4.  The logical chunk it holds is the same for every i.
+        const int ca = (lane % 8) ^ ((4 * wave + lane / 16) % 8);
+        const int cb = (lane % 4) ^ (lane / 16);
+        const f16* asrc[NA];
+        const int8_t* bsrc[NB];
 #pragma unroll
-        for (int pp = 0; pp < 2; ++pp) {
-            f16x8 bf[2][TJ];
+        for (int i = 0; i < NA; ++i)
+            asrc[i] = a.x + min(m0 + (NT * i + 64 * wave + lane) / 8, a.M - 1) * a.ldx + 8 * ca;
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                const u32x4 q = *reinterpret_cast<const u32x4*>(bs + 32 * j * KT + 16 * ((2 * pp + h) ^ swb));
-                uint32_t o[8];
-                i8x4_to_f16(q.x, o[0], o[1]);
-                i8x4_to_f16(q.y, o[2], o[3]);
-                i8x4_to_f16(q.z, o[4], o[5]);
-                i8x4_to_f16(q.w, o[6], o[7]);
-                bf[0][j] = __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
-                bf[1][j] = __builtin_bit_cast(f16x8, u32x4{o[4], o[5], o[6], o[7]});
-            }
+        for (int i = 0; i < NB; ++i)
+            bsrc[i] = (const int8_t*)a.w + min(n0 + (NT * i + 64 * wave + lane) / 4, a.N - 1) * a.ldw + 16 * cb;
+        auto dma = [&](int kt, int buf) {
+            const int k0 = min(kt, ktiles - 1) * KT;  // past the end: re-reads the last tile
+            uint8_t* st = smem + buf * (ASZ + BSZ);
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int c = 16 * ((4 * pp + 2 * h + e) ^ swa);
+            for (int i = 0; i < NA; ++i) lds_dma16(asrc[i] + k0, st + 16 * (NT * i + 64 * wave));
 #pragma unroll
-                for (int i = 0; i < TI; ++i) {
-                    const f16x8 af = *reinterpret_cast<const f16x8*>(as + 32 * i * (KT * 2) + c);
+            for (int i = 0; i < NB; ++i) lds_dma16(bsrc[i] + k0, st + ASZ + 16 * (NT * i + 64 * wave));
+        };
+
+        // this lane's rows: activation rows wm WM + 32 i + r32 (swizzle (row / 2) % 8 = (r32 / 2) % 8
+        // since WM and 32 are multiples of 16), weight rows wn WN + 32 j + r32 (swizzle (r32 / 4) % 4)
+        const int swa = (r32 / 2) % 8, swb = (r32 / 4) % 4;
+        auto mfmas = [&](int buf) {
+            const uint8_t* as = smem + buf * (ASZ + BSZ) + (wm * WM + r32) * (KT * 2);
+            const uint8_t* bs = smem + buf * (ASZ + BSZ) + ASZ + (wn * WN + r32) * KT;
 #pragma unroll
-                    for (int j = 0; j < TJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[e][j], acc[i][j], 0, 0, 0);
+            for (int pp = 0; pp < 2; ++pp) {
+                f16x8 bf[2][TJ];
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) {
+                    const u32x4 q = *reinterpret_cast<const u32x4*>(bs + 32 * j * KT + 16 * ((2 * pp + h) ^ swb));
+                    uint32_t o[8];
+                    i8x4_to_f16(q.x, o[0], o[1]);
+                    i8x4_to_f16(q.y, o[2], o[3]);
+                    i8x4_to_f16(q.z, o[4], o[5]);
+                    i8x4_to_f16(q.w, o[6], o[7]);
+                    bf[0][j] = __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
+                    bf[1][j] = __builtin_bit_cast(f16x8, u32x4{o[4], o[5], o[6], o[7]});
+                }
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int c = 16 * ((4 * pp + 2 * h + e) ^ swa);
+#pragma unroll
+                    for (int i = 0; i < TI; ++i) {
+                        const f16x8 af = *reinterpret_cast<const f16x8*>(as + 32 * i * (KT * 2) + c);
+#pragma unroll
+                        for (int j = 0; j < TJ; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[e][j], acc[i][j], 0, 0, 0);
+                    }
                 }
             }
-        }
-    };
+        };
 
-    // Barrier without a memory fence: the DMA data a wave needs is covered by its wait_vmcnt, and
-    // the loop writes LDS only by DMA; the fragment reads of a buffer complete before the barrier
-    // after which the next DMA may overwrite it.
-    constexpr int ND = NA + NB;
+        // Barrier without a memory fence: the DMA data a wave needs is covered by its wait_vmcnt, and
+        // the loop writes LDS only by DMA; the fragment reads of a buffer complete before the barrier
+        // after which the next DMA may overwrite it.
+        constexpr int ND = NA + NB;
 #pragma unroll
-    for (int st = 0; st < STAGES - 1; ++st) dma(st, st);
-    wait_vmcnt<(STAGES - 2) * ND>();
-    __builtin_amdgcn_s_barrier();
-    // unrolled by STAGES: every stage buffer index is a constant (1-2% faster on the A8 configs)
-    for (int k0 = 0; k0 < ktiles; k0 += STAGES) {
+        for (int st = 0; st < STAGES - 1; ++st) dma(st, st);
+        wait_vmcnt<(STAGES - 2) * ND>();
+        __builtin_amdgcn_s_barrier();
+        // unrolled by STAGES: every stage buffer index is a constant (1-2% faster on the A8 configs)
+        for (int k0 = 0; k0 < ktiles; k0 += STAGES) {
 #pragma unroll
-        for (int s = 0; s < STAGES; ++s) {
-            const int kt = k0 + s;
-            if (kt >= ktiles) break;
-            dma(kt + STAGES - 1, (s + STAGES - 1) % STAGES);
-            __builtin_amdgcn_sched_barrier(0);
-            mfmas(s);
-            wait_lgkmcnt0();
-            wait_vmcnt<(STAGES - 2) * ND>();  // tile kt + 1 has landed
-            __builtin_amdgcn_s_barrier();
+            for (int s = 0; s < STAGES; ++s) {
+                const int kt = k0 + s;
+                if (kt >= ktiles) break;
+                dma(kt + STAGES - 1, (s + STAGES - 1) % STAGES);
+                __builtin_amdgcn_sched_barrier(0);
+                mfmas(s);
+                wait_lgkmcnt0();
+                wait_vmcnt<(STAGES - 2) * ND>();  // tile kt + 1 has landed
+                __builtin_amdgcn_s_barrier();
+            }
         }
+        wait_vmcnt<0>();
     }
-    wait_vmcnt<0>();
 
     // Epilogue: y = ldexp(acc, xexp[m]) * scale[n] + bias[n], staged through LDS in passes of RP
     // rows (row stride BNT + 8 words); every thread writes 8 consecutive outputs with 16-byte stores.
@@ -757,6 +766,87 @@ __global__ __launch_bounds__(512) void gemm_wo_dma_kernel(GemmF16Args a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[q][e] = __builtin_ldexpf(e < 4 ? v0[e] : v1[e - 4], e2) * cs[e] + bv[e];
             }
+        }
+        int64_t mq[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) mq[q] = m0 + pass * RP + tid / CPR + (NT / CPR) * q;
+        if (a.res.r) residual_apply8<Q>(a.res, mq, nc, a.M, a.N, rsv, v);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int64_t m = mq[q];
+            if (m < a.M && ncount > 0) store8_rt(a.y, a.y_dtype, m * a.ldy + nc, v[q], ncount, vec);
+        }
+    }
+}
+
+// 256 x 256 tiles over a decoded GGUF tensor (fp16 w 2^-wexp[n]): the main loop of gemm_pp.h, then y =
+// ldexp(acc, xexp[m] + wexp[n]) + bias[n], with a residual as in gemm_wo_dma_kernel.
+__global__ __launch_bounds__(512) void gemm_f16pp_kernel(GemmF16Args a) {
+    constexpr int NT = 512, BT = 256;
+    using Loop = PingPong<false>;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[Loop::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 2, wn = wave & 3, r16 = lane & 15, g = lane >> 4;
+    int mt, nt;
+    xcd_tile_f16(blockIdx.x, (int)gridDim.x, (int)((a.M + BT - 1) / BT), (int)((a.N + BT - 1) / BT), mt, nt);
+    const int64_t n0 = (int64_t)nt * BT, m0 = (int64_t)mt * BT;
+    f32x4 acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Loop::run(smem, (const uint8_t*)(a.x + m0 * a.ldx), a.ldx * 2, (int)min<int64_t>(BT, a.M - m0),
+              (const uint8_t*)((const f16*)a.w + n0 * a.ldw), a.ldw * 2, (int)min<int64_t>(BT, a.N - n0), (int)(a.K / 64), tid, acc);
+
+    // Epilogue, in passes of 64 rows through LDS: as in gemm_wo_dma_kernel, every operand is requested
+    // before the first store, each pass computes all of a thread's outputs before its stores, and the
+    // passes synchronize LDS only.
+    constexpr int ORW = BT + 8, CPR = BT / 8, RP = 64, Q = RP * CPR / NT;
+    static_assert(RP * ORW * 4 + BT * 4 <= Loop::LDS, "output staging must fit");
+    float* ot = reinterpret_cast<float*>(smem);
+    int* erow = reinterpret_cast<int*>(smem + Loop::LDS - BT * 4);
+    const int cc = tid % CPR;
+    const int64_t nc = n0 + 8 * cc;
+    const int ncount = (int)max<int64_t>(0, min<int64_t>(8, a.N - nc));
+    const int xer = a.xexp ? a.xexp[min(m0 + min(tid, BT - 1), (int64_t)a.M - 1)] : 0;
+    int we[8];
+    uint32_t bvb[8], rsb[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int64_t n = min(nc + e, a.N - 1);
+        we[e] = a.wexp[n];
+        bvb[e] = a.bias ? load_bits_rt(a.bias, a.bias_dtype, n) : 0u;
+    }
+    residual_scale_bits8(a.res, nc, a.N, rsb);
+    const bool vec = (a.ldy % 8 == 0) && ((uintptr_t)a.y % 16 == 0);
+    lds_barrier();  // every wave is past the main loop, its DMAs included
+    if (tid < BT) erow[tid] = xer;
+    float bv[8], rsv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bv[e] = a.bias ? bits_to_f32_rt(bvb[e], a.bias_dtype) : 0.0f;
+    residual_scales8(a.res, rsb, rsv);
+#pragma unroll
+    for (int pass = 0; pass < BT / RP; ++pass) {
+        if (pass) lds_barrier();  // the previous pass is no longer read
+        if (wm == pass / 2) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        ot[(16 * i + 4 * g + r) * ORW + 64 * wn + 16 * j + r16] = acc[4 * (pass % 2) + i][j][r];
+        }
+        lds_barrier();
+        float v[Q][8];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int row = tid / CPR + (NT / CPR) * q;
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(ot + row * ORW + 8 * cc);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(ot + row * ORW + 8 * cc + 4);
+            const int xe = erow[pass * RP + row];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[q][e] = __builtin_ldexpf(e < 4 ? v0[e] : v1[e - 4], xe + we[e]) + bv[e];
         }
         int64_t mq[Q];
 #pragma unroll
@@ -1026,6 +1116,25 @@ __global__ __launch_bounds__((64 * wo_dmas_waves<BMT, BNT, KT>())) void gemm_wo_
     }
 }
 
+// The main loops of gemm_pp.h hold 32-bit byte offsets of a tile's 256 rows.
+inline bool pp_strides(const GemmF16Args& a) { return a.ldx <= (1 << 22) && a.ldw <= (1 << 22); }
+
+// The 256 x 256 INT8 kernel by LoRA dtype; rows of whole weight half-tiles take the two-group loop.
+hipError_t launch_wo256(dim3 grid, const GemmF16Args& a, hipStream_t st) {
+    auto go = [&]<int LDU>() {
+        if (a.K % 128 == 0 && pp_strides(a)) hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3, LDU, true>), grid, dim3(512), 0, st, a);
+        else hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3, LDU>), grid, dim3(512), 0, st, a);
+        return hipGetLastError();
+    };
+    if (!a.lora.t) return go.template operator()<-1>();
+    switch (a.lora.up_dt) {
+        case DT_BF16: return go.template operator()<DT_BF16>();
+        case DT_F16: return go.template operator()<DT_F16>();
+        case DT_F32: return go.template operator()<DT_F32>();
+    }
+    return hipErrorInvalidValue;
+}
+
 template <int WK, int GT>
 hipError_t launch1(const GemmF16Args& a, hipStream_t st) {
     if (a.y_dtype != DT_F32 && a.y_dtype != DT_F16 && a.y_dtype != DT_BF16) return hipErrorInvalidValue;
@@ -1047,18 +1156,12 @@ hipError_t launch1(const GemmF16Args& a, hipStream_t st) {
                 rest.y = (uint8_t*)a.y + m1 * a.ldy * dt_bytes(a.y_dtype);
                 if (a.res.r) rest.res.r = (const uint8_t*)a.res.r + m1 * a.res.ldr * dt_bytes(a.res.r_dt);
                 auto tiles_of = [](const GemmF16Args& g, int bm) { return ((g.M + bm - 1) / bm) * ((g.N + 255) / 256); };
-                hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3>), dim3((unsigned)tiles_of(top, 256)), dim3(512), 0, st, top);
-                const hipError_t err = hipGetLastError();
+                const hipError_t err = launch_wo256(dim3((unsigned)tiles_of(top, 256)), top, st);
                 if (err != hipSuccess) return err;
                 hipLaunchKernelGGL((gemm_wo_dma_kernel<128, 3>), dim3((unsigned)tiles_of(rest, 128)), dim3(512), 0, st, rest);
                 return hipGetLastError();
             }
-            if (!a.lora.t) hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3>), grid, dim3(512), 0, st, a);
-            else if (a.lora.up_dt == DT_BF16) hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3, DT_BF16>), grid, dim3(512), 0, st, a);
-            else if (a.lora.up_dt == DT_F16) hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3, DT_F16>), grid, dim3(512), 0, st, a);
-            else if (a.lora.up_dt == DT_F32) hipLaunchKernelGGL((gemm_wo_dma_kernel<256, 3, DT_F32>), grid, dim3(512), 0, st, a);
-            else return hipErrorInvalidValue;
-            return hipGetLastError();
+            return launch_wo256(grid, a, st);
         }
         if (a.lora.t) return hipErrorInvalidValue;  // only the 256 x 256 DMA kernel adds a LoRA term
         // grids of fewer than 160 tiles of 128 x 128: small tiles through a DMA ring, the one of
@@ -1111,6 +1214,13 @@ hipError_t launch1(const GemmF16Args& a, hipStream_t st) {
                          (uintptr_t)a.w % 16 == 0;
         if (vec) {
             auto tiles = [&](int bm, int bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+            // From 96 tiles of 256 x 256 (a third of the CUs) they beat the smaller tiles of the ring kernel
+            // (Q4_K, us: M2048 K = N = 3072, 96 tiles, 79.6 against 82.7; M1536 K = N = 4096, 96, 97 / 105;
+            // M2048, 128, 100 / 116; M1024 K5120 N13824, 216, 158 / 253; below, M1024 K = N = 4096, 64, 95 / 69).
+            if (tiles(256, 256) >= 96 && pp_strides(a)) {
+                hipLaunchKernelGGL(gemm_f16pp_kernel, dim3((unsigned)tiles(256, 256)), dim3(512), 0, st, a);
+                return hipGetLastError();
+            }
             int bm = 128, bn = 128;
             if (tiles(128, 128) < 256) {
                 int64_t best = 0;

@@ -13,6 +13,7 @@
 #include "qlin_internal.h"
 #include "lora_frag.h"
 #include "prologue_dev.h"
+#include "gemm_pp.h"
 
 namespace qlin {
 namespace {
@@ -1039,6 +1040,122 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_i8dma_kernel(GemmI8Args p
     }
 }
 
+// 256 x 256 tiles over the decoded int8 grid: the main loop of gemm_pp.h, then the epilogue of
+// gemm_i8dma_kernel, in passes of 64 rows.  us of this kernel against the 32 x 32 loop with one barrier a
+// k-tile that it replaces: PPTIMES
+template <int LDU = -1>
+__global__ __launch_bounds__(512) void gemm_i8pp_kernel(GemmI8Args p, const int8_t* __restrict__ w8) {
+    constexpr int NT = 512, BT = 256;
+    using Loop = PingPong<true>;
+    constexpr int RC = lora_max_rank<LDU < 0 ? DT_BF16 : LDU, BT, BT>(Loop::LDS);  // LoRA ranks staged at once
+    static_assert(LDU < 0 || RC >= i8dma_lora_rank(LDU), "the host's rank limit must fit every tile shape");
+    constexpr int SM = Loop::LDS + BT * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[SM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 2, wn = wave & 3, r16 = lane & 15, g = lane >> 4;
+    int mt, nt;
+    xcd_tile(blockIdx.x, (int)gridDim.x, (int)((p.M + BT - 1) / BT), (int)((p.N + BT - 1) / BT), mt, nt);
+    const int64_t n0 = (int64_t)nt * BT, m0 = (int64_t)mt * BT;
+    i32x4 acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+    Loop::run(smem, (const uint8_t*)p.xq + m0 * p.ldx, p.ldx, (int)min<int64_t>(BT, p.M - m0), (const uint8_t*)w8 + n0 * p.K, p.K,
+              (int)min<int64_t>(BT, p.N - n0), (int)(p.K / 128), tid, acc);
+
+    constexpr int ORW = BT + 8, CPR = BT / 8, RP = 64, Q = RP * CPR / NT;
+    static_assert(RP * ORW * 4 + BT * 4 <= SM, "output staging must fit");
+    int32_t* ot = reinterpret_cast<int32_t*>(smem);
+    float* srow = reinterpret_cast<float*>(smem + SM - BT * 4);
+    const int cc = tid % CPR;
+    const int64_t nc = n0 + 8 * cc;
+    const int ncount = (int)max<int64_t>(0, min<int64_t>(8, p.N - nc));
+    const float sxr = p.sx[min(m0 + min(tid, BT - 1), (int64_t)p.M - 1)];
+    constexpr int CB8 = LDU >= 0 ? 1 : 8;  // with a LoRA term the staged values are final
+    float sc[CB8];
+    uint32_t bvb[CB8], rsb[8];
+    // ((f32(acc) * sx) * s_channel) + bias, each operation rounded on its own
+    auto finish = [&](int c, float sx, float sn, float bias) {
+#pragma clang fp contract(off)
+        float val = (float)c * sx;
+        val = val * sn;
+        if (p.bias) val = val + bias;
+        return val;
+    };
+    if constexpr (LDU < 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t n = min(nc + e, p.N - 1);
+            sc[e] = p.s_ch[n];
+            bvb[e] = p.bias ? load_bits_rt(p.bias, p.bias_dtype, n) : 0u;
+        }
+    }
+    residual_scale_bits8(p.res, nc, p.N, rsb);
+    const bool vec = (p.ldy % 8 == 0) && ((uintptr_t)p.y % 16 == 0);
+    lds_barrier();  // every wave is past the main loop, its DMAs included
+    if (tid < BT) srow[tid] = sxr;
+    if constexpr (LDU >= 0) {
+        float scn[4];
+        uint32_t bvj[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t n = min(n0 + 64 * wn + 16 * j + r16, p.N - 1);
+            scn[j] = p.s_ch[n];
+            bvj[j] = p.bias ? load_bits_rt(p.bias, p.bias_dtype, n) : 0u;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float bvn = p.bias ? bits_to_f32_rt(bvj[j], p.bias_dtype) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc[i][j][r] = __float_as_int(finish(acc[i][j][r], srow[128 * wm + 16 * i + 4 * g + r], scn[j], bvn));
+        }
+        lora_tile_epilogue_ranks<LDU, BT, BT, RC, NT, 8, 4>(p.lora, smem, m0, n0, p.M, p.N, 128 * wm, 64 * wn, tid, lane, acc);
+    }
+    float rsv[8];
+    residual_scales8(p.res, rsb, rsv);
+#pragma unroll
+    for (int pass = 0; pass < BT / RP; ++pass) {
+        if (pass) lds_barrier();  // the previous pass is no longer read
+        if (wm == pass / 2) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        ot[(16 * i + 4 * g + r) * ORW + 64 * wn + 16 * j + r16] = acc[4 * (pass % 2) + i][j][r];
+        }
+        lds_barrier();
+        float v[Q][8];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int row = tid / CPR + (NT / CPR) * q;
+            const i32x4 a0 = *reinterpret_cast<const i32x4*>(ot + row * ORW + 8 * cc);
+            const i32x4 a1 = *reinterpret_cast<const i32x4*>(ot + row * ORW + 8 * cc + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int c = e < 4 ? a0[e] : a1[e - 4];
+                if constexpr (LDU >= 0) v[q][e] = __int_as_float(c);
+                else v[q][e] = finish(c, srow[pass * RP + row], sc[e], p.bias ? bits_to_f32_rt(bvb[e], p.bias_dtype) : 0.0f);
+            }
+        }
+        int64_t mq[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) mq[q] = m0 + pass * RP + tid / CPR + (NT / CPR) * q;
+        if (p.res.r) residual_apply8<Q>(p.res, mq, nc, p.M, p.N, rsv, v);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int64_t m = mq[q];
+            if (m < p.M && ncount > 0) store8_rt(p.y, p.y_dtype, m * p.ldy + nc, v[q], ncount, vec);
+        }
+    }
+}
+
 // A8 linear for few activation rows (up to 32): weight streaming, the decode in the load stage.
 // One 512-thread workgroup per 16 weight rows; the K range is split across the 8 waves in stages
 // of 256 values.  In a stage, lane l decodes the 64 codes k = 64 (l / 16) .. + 63 of weight row
@@ -1218,16 +1335,22 @@ hipError_t launch_o(const GemmI8Args& p, hipStream_t st) {
             rest.y = (uint8_t*)p.y + m1 * p.ldy * dt_bytes(p.y_dtype);
             if (p.res.r) rest.res.r = (const uint8_t*)p.res.r + m1 * p.res.ldr * dt_bytes(p.res.r_dt);
             auto tiles_of = [](const GemmI8Args& g, int bm) { return ((g.M + bm - 1) / bm) * ((g.N + 255) / 256); };
-            hipLaunchKernelGGL((gemm_i8dma_kernel<256, 256, 128, 2, false>), dim3((unsigned)tiles_of(top, 256)), dim3(512), 0,
-                               st, top, top.w8);
+            hipLaunchKernelGGL(gemm_i8pp_kernel<>, dim3((unsigned)tiles_of(top, 256)), dim3(512), 0, st, top, top.w8);
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) return err;
             hipLaunchKernelGGL((gemm_i8dma_kernel<128, 256, 128, 2, false>), dim3((unsigned)tiles_of(rest, 128)), dim3(512),
                                0, st, rest, rest.w8);
             return hipGetLastError();
         }
-        if (tiles(256, 256) >= 192)
-            go.template operator()<256, 256>();
+        if (tiles(256, 256) >= 192) {
+            const dim3 grid((unsigned)tiles(256, 256));
+            switch (ldu) {
+                case -1: hipLaunchKernelGGL(gemm_i8pp_kernel<>, grid, dim3(512), 0, st, p, p.w8); break;
+                case DT_BF16: hipLaunchKernelGGL(gemm_i8pp_kernel<DT_BF16>, grid, dim3(512), 0, st, p, p.w8); break;
+                case DT_F16: hipLaunchKernelGGL(gemm_i8pp_kernel<DT_F16>, grid, dim3(512), 0, st, p, p.w8); break;
+                case DT_F32: hipLaunchKernelGGL(gemm_i8pp_kernel<DT_F32>, grid, dim3(512), 0, st, p, p.w8); break;
+            }
+        }
         // 128 x 160 tiles (2 x 5 waves, no LoRA term) when they make one round of at least 3/4 of
         // the 256 CUs and 256 x 256 tiles would not fill the GPU (M1024 N5120: 256 of them)
         else if (ldu == -1 && tiles(128, 160) >= 192 && tiles(128, 160) <= 256) {

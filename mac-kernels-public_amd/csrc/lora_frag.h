@@ -131,7 +131,8 @@ __device__ __forceinline__ void mfma_raw(const Raw8<DA>& ra, const Raw8<DB>& rb,
 // acc[i][j] (fp32 values, or their bits in int32 registers), so the base value is the MFMAs'
 // accumulator input.  A wave's sub-tile (i, j) covers tile rows wr0 + 32 i .. + 31 and columns
 // wc0 + 32 j .. + 31, in the MFMA C layout (lane l, register r: row 8 (r / 4) + 4 (l / 32) + r % 4,
-// column l % 32).  LDS rows are unpadded; their 16-byte chunks are XOR-swizzled (lora_chunk) so the
+// column l % 32); with four-register accumulators, sub-tiles of 16 x 16 (row 4 (l / 16) + r, column
+// l % 16).  LDS rows are unpadded; their 16-byte chunks are XOR-swizzled (lora_chunk) so the
 // 32 rows of a fragment read spread over the banks.  Requires 8 <= R <= RC, R % 8 == 0 and 16-byte
 // aligned t and up rows (t row stride R); lds must hold lora_lds_bytes<DU, BMT, BNT, RC>().  No loop
 // here has a run-time trip count, so the caller's accumulators stay in registers.  Starts and ends
@@ -160,8 +161,16 @@ __device__ __forceinline__ int lora_chunk(int row, int c) {
 template <int DU, int BMT, int BNT, int RC, int NT, int TI, int TJ, bool PARTS, typename AccT>
 __device__ __forceinline__ void lora_tile_epilogue(const LoraTile& L, uint8_t* lds, int64_t m0, int64_t n0, int64_t M,
                                                    int64_t N, int wr0, int wc0, int tid, int lane, AccT (&acc)[TI][TJ]) {
-    static_assert(sizeof(AccT) == sizeof(f32x16), "32 x 32 accumulators: fp32 values or their int32 bits");
-    static_assert(RC % 16 == 0, "whole MFMA steps");
+    constexpr bool M16 = sizeof(AccT) == sizeof(f32x4);
+    static_assert(M16 || sizeof(AccT) == sizeof(f32x16), "accumulators: fp32 values or their int32 bits");
+    // sub-tile size, ranks per MFMA, and the 8-rank chunks of one that a lane's fragment comes from
+    constexpr int SUB = M16 ? 16 : 32, KS = M16 ? 32 : 16, CS = KS / 8;
+    static_assert(RC % KS == 0, "whole MFMA steps");
+    using CT = std::conditional_t<M16, f32x4, f32x16>;
+    auto mfma = [](bf16x8 a, bf16x8 b, CT c) {
+        if constexpr (M16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+        else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    };
     constexpr int ES = DU == DT_F32 ? 4 : 2, UPP = 16 / ES;   // up element size, elements per 16 bytes
     constexpr int TBPR = RC * 2, UBPR = RC * ES;             // bytes per LDS row: t hi (or lo), up
     constexpr int TP = BMT * RC / 8 / NT, UP = BNT * RC / UPP / NT;  // pieces per thread: 8 t, 16 B of up
@@ -170,7 +179,7 @@ __device__ __forceinline__ void lora_tile_epilogue(const LoraTile& L, uint8_t* l
     uint8_t* th = lds;
     uint8_t* tl = lds + BMT * TBPR;
     uint8_t* us = lds + 2 * BMT * TBPR;
-    const int r32 = lane & 31, h = lane >> 5;
+    const int rs = lane % SUB, h = lane / SUB;
     float tv[TP][8];
     u32x4 uv[UP];
     const int64_t ldt = L.ld_t ? L.ld_t : L.R;
@@ -230,16 +239,16 @@ __device__ __forceinline__ void lora_tile_epilogue(const LoraTile& L, uint8_t* l
     // compile-time block indices, so that every access to the caller's accumulators is constant
     auto col = [&]<int J>() {
         __builtin_amdgcn_sched_barrier(0);
-        const int un = wc0 + 32 * J + r32;
-        bf16x8 bh[RC / 16], bl[RC / 16];
+        const int un = wc0 + SUB * J + rs;
+        bf16x8 bh[RC / KS], bl[RC / KS];
 #pragma unroll
-        for (int q = 0; q < RC / 16; ++q) {
+        for (int q = 0; q < RC / KS; ++q) {
             Raw8<DU> rb;
             if constexpr (DU == DT_F32) {
-                rb.v[0] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, 4 * q + 2 * h));
-                rb.v[1] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, 4 * q + 2 * h + 1));
+                rb.v[0] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, 2 * (CS * q + h)));
+                rb.v[1] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, 2 * (CS * q + h) + 1));
             } else {
-                rb.v[0] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, 2 * q + h));
+                rb.v[0] = *reinterpret_cast<const u32x4*>(us + lora_chunk<UBPR>(un, CS * q + h));
             }
             if constexpr (SU) {
                 float f[8];
@@ -251,15 +260,15 @@ __device__ __forceinline__ void lora_tile_epilogue(const LoraTile& L, uint8_t* l
         }
         auto row = [&]<int I>() {
             __builtin_amdgcn_sched_barrier(0);
-            const int tm = wr0 + 32 * I + r32;
-            f32x16 c = __builtin_bit_cast(f32x16, acc[I][J]);
+            const int tm = wr0 + SUB * I + rs;
+            CT c = __builtin_bit_cast(CT, acc[I][J]);
 #pragma unroll
-            for (int q = 0; q < RC / 16; ++q) {
-                const bf16x8 ah = *reinterpret_cast<const bf16x8*>(th + lora_chunk<TBPR>(tm, 2 * q + h));
-                const bf16x8 al = *reinterpret_cast<const bf16x8*>(tl + lora_chunk<TBPR>(tm, 2 * q + h));
-                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[q], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[q], c, 0, 0, 0);
-                if constexpr (SU) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[q], c, 0, 0, 0);
+            for (int q = 0; q < RC / KS; ++q) {
+                const bf16x8 ah = *reinterpret_cast<const bf16x8*>(th + lora_chunk<TBPR>(tm, CS * q + h));
+                const bf16x8 al = *reinterpret_cast<const bf16x8*>(tl + lora_chunk<TBPR>(tm, CS * q + h));
+                c = mfma(ah, bh[q], c);
+                c = mfma(al, bh[q], c);
+                if constexpr (SU) c = mfma(ah, bl[q], c);
             }
             acc[I][J] = __builtin_bit_cast(AccT, c);
         };

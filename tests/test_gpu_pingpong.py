@@ -1,0 +1,69 @@
+"""The 256 x 256 tile GEMMs whose two wave groups take turns: contractions of one k-tile up (an odd and an
+even number of them, fewer than the pipeline is deep), ragged last tiles in both directions.
+
+fp16 operands are exact here (small integers times powers of two), so the weight-only outputs differ
+from the float64 product by the fp32 sum alone: 1e-6 of it relative to |x| |w|.  The A8 output is
+replayed exactly: the int8 products summed in float64, then the epilogue's fp32 steps.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _ints(shape, lo, hi, seed):
+    return torch.randint(lo, hi + 1, shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+def _check(y, x, w, extra=None):
+    want = x.double() @ w.double().T
+    bound = x.double().norm(dim=1, keepdim=True) * w.double().norm(dim=1) + 1e-30
+    if extra is not None:
+        want = want + extra
+    assert ((y.double() - want).abs() / bound).max().item() < 1e-6
+
+
+@pytest.mark.parametrize("m,n", [(2305, 2600), (600, 8200)])  # 110 and 99 tiles, last ones 1 row, 40 and 88 x 8
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 1088])
+def test_decoded_gguf(k, m, n):
+    import qlin
+    x = _ints((m, k), -8, 8, k).half()
+    q = _ints((n, k), -127, 127, m).to(torch.int8)
+    d = torch.full((n, k // 32, 1), 2.0 ** -7, dtype=torch.float16, device=DEV)
+    raw = torch.cat([d.view(torch.uint8), q.view(n, k // 32, 32).view(torch.uint8)], 2).reshape(n, -1).contiguous()
+    r = _ints((m, n), -4, 4, 7).float()
+    y = qlin.gguf_linear(x, raw, "Q8_0", (n, k), out_dtype=torch.float32)
+    _check(y, x, q.float() / 128)
+    y = qlin.gguf_linear(x, raw, "Q8_0", (n, k), out_dtype=torch.float32, residual=r)
+    _check(y, x, q.float() / 128, r.double())
+
+
+@pytest.mark.parametrize("m,n", [(3329, 3000), (513, 14000)])  # 168 and 165 tiles
+@pytest.mark.parametrize("k", [64, 128, 256, 384, 640, 1152])  # 64: rows of half a weight half-tile
+def test_int8(k, m, n):
+    import qlin
+    x = _ints((m, k), -8, 8, k).half()
+    q = _ints((n, k), -128, 127, m).to(torch.int8)
+    y = qlin.int8_linear(x, q, torch.full((n,), 0.5, device=DEV), out_dtype=torch.float32)
+    _check(y, x, q.float() / 2)
+
+
+@pytest.mark.parametrize("m,n", [(3585, 3500), (600, 16400)])  # 210 and 195 tiles
+@pytest.mark.parametrize("bits,k", [(4, 128), (6, 256), (4, 384), (6, 640)])
+def test_a8(bits, k, m, n):
+    import qlin
+    from qlin.quantize import pack_codes
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(m, k, generator=g).half().to(DEV)
+    codes = torch.randint(1, 1 << bits, (n, k), generator=g)
+    packed = pack_codes(codes, bits).to(DEV)
+    s_rel = (1 + 3 * torch.rand(n, k // 64, generator=g)).half().to(DEV)
+    s_ch = (torch.rand(n, generator=g) * 1e-2).to(DEV)
+    bias = torch.randn(n, generator=g).to(DEV)
+    y = qlin.w4a8_int8_linear(x, packed, s_rel, s_ch, None, None, bias, 64, 128)
+    q, sx = qlin.quantize_int8_rowwise(x, 128)
+    acc = q.double() @ qlin.w4a8_int8_grid(packed, s_rel, None, 64).double().T
+    want = ((acc.float() * sx) * s_ch + bias).half()
+    assert torch.equal(y, want)
