@@ -1317,25 +1317,26 @@ hipError_t run_gemm_f16(const GemmF16Args& a, hipStream_t st) {
 // One workgroup per weight row n: the row's exponent e[n] (of its largest |w|, as
 // gguf_row_exp_kernel computes it) and the row stored as fp16(w 2^-e[n]), 8 values per 16-byte
 // store.  CPT > 0: the packed row is first copied to LDS in dwords (the decode's byte reads then
-// hit LDS, not the texture path), and each thread decodes its CPT chunks of 8 values (chunk c at
-// 8 (tid + 256 c)) once and keeps them in registers (K <= 2048 CPT); CPT = 0: any K, the row
-// decoded twice from global memory (the second time from cache).
-template <int T, int CPT>
-__global__ __launch_bounds__(256) void gguf_decode_f16_kernel(const uint8_t* __restrict__ w, int64_t row_bytes,
+// hit LDS, not the texture path), and each of the NT threads decodes its CPT chunks of 8 values (chunk c
+// at 8 (tid + NT c)) once and keeps them in registers (K <= 8 NT CPT); CPT = 0: any K, the row
+// decoded twice from global memory (the second time from cache), which byte reads and the second decode
+// bound: Q6_K K12288 N3072 101 us that way, 38 us with 512 threads of 4 chunks (107 MB moved).
+template <int T, int CPT, int NT = 256>
+__global__ __launch_bounds__(NT) void gguf_decode_f16_kernel(const uint8_t* __restrict__ w, int64_t row_bytes,
                                                               int64_t K, int32_t* __restrict__ wexp,
                                                               f16* __restrict__ out) {
     constexpr int QK = gguf::Info<T>::QK, TS = gguf::Info<T>::TS;
-    constexpr int RW = CPT > 0 ? (CPT * 2048 / QK * TS + 3) / 4 : 1;  // dwords of the longest row
-    __shared__ float red[4];
+    constexpr int RW = CPT > 0 ? (CPT * NT * 8 / QK * TS + 3) / 4 : 1;  // dwords of the longest row
+    __shared__ float red[NT / 64];
     __shared__ uint32_t rs[RW];
     const int64_t n = blockIdx.x;
     const uint8_t* row = w + n * row_bytes;
     if constexpr (CPT > 0) {
         if ((((uintptr_t)w | (uintptr_t)row_bytes) & 3) == 0) {
             const uint32_t* r4 = reinterpret_cast<const uint32_t*>(row);
-            for (int i = threadIdx.x; i < row_bytes / 4; i += 256) rs[i] = r4[i];
+            for (int i = threadIdx.x; i < row_bytes / 4; i += NT) rs[i] = r4[i];
         } else {
-            for (int i = threadIdx.x; i < row_bytes; i += 256) reinterpret_cast<uint8_t*>(rs)[i] = row[i];
+            for (int i = threadIdx.x; i < row_bytes; i += NT) reinterpret_cast<uint8_t*>(rs)[i] = row[i];
         }
         __syncthreads();
         row = reinterpret_cast<const uint8_t*>(rs);
@@ -1357,7 +1358,7 @@ __global__ __launch_bounds__(256) void gguf_decode_f16_kernel(const uint8_t* __r
     if constexpr (CPT > 0) {
 #pragma unroll
         for (int c = 0; c < CPT; ++c) {
-            const int64_t j = ((int64_t)threadIdx.x + 256 * c) * 8;
+            const int64_t j = ((int64_t)threadIdx.x + NT * c) * 8;
             if (j < K) decode(j, v[c]);
             else
 #pragma unroll
@@ -1366,7 +1367,7 @@ __global__ __launch_bounds__(256) void gguf_decode_f16_kernel(const uint8_t* __r
             for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf(v[c][t]));
         }
     } else {
-        for (int64_t j = (int64_t)threadIdx.x * 8; j < K; j += 256 * 8) {
+        for (int64_t j = (int64_t)threadIdx.x * 8; j < K; j += NT * 8) {
             decode(j, v[0]);
 #pragma unroll
             for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf(v[0][t]));
@@ -1375,16 +1376,19 @@ __global__ __launch_bounds__(256) void gguf_decode_f16_kernel(const uint8_t* __r
     amax = wave_max(amax);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
     __syncthreads();
-    const int e = frexp_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    amax = red[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; ++i) amax = fmaxf(amax, red[i]);
+    const int e = frexp_exp(amax);
     if (threadIdx.x == 0) wexp[n] = e;
     if constexpr (CPT > 0) {
 #pragma unroll
         for (int c = 0; c < CPT; ++c) {
-            const int64_t j = ((int64_t)threadIdx.x + 256 * c) * 8;
+            const int64_t j = ((int64_t)threadIdx.x + NT * c) * 8;
             if (j < K) store(j, v[c], e);
         }
     } else {
-        for (int64_t j = (int64_t)threadIdx.x * 8; j < K; j += 256 * 8) {
+        for (int64_t j = (int64_t)threadIdx.x * 8; j < K; j += NT * 8) {
             decode(j, v[0]);
             store(j, v[0], e);
         }
@@ -1402,6 +1406,7 @@ hipError_t run_gguf_decode_f16(int type, const uint8_t* w, int64_t row_bytes, in
         if (cpt <= 1) hipLaunchKernelGGL((gguf_decode_f16_kernel<T, 1>), grid, block, 0, st, w, row_bytes, K, e, out);
         else if (cpt <= 2) hipLaunchKernelGGL((gguf_decode_f16_kernel<T, 2>), grid, block, 0, st, w, row_bytes, K, e, out);
         else if (cpt <= 4) hipLaunchKernelGGL((gguf_decode_f16_kernel<T, 4>), grid, block, 0, st, w, row_bytes, K, e, out);
+        else if (cpt <= 8) hipLaunchKernelGGL((gguf_decode_f16_kernel<T, 4, 512>), grid, dim3(512), 0, st, w, row_bytes, K, e, out);
         else hipLaunchKernelGGL((gguf_decode_f16_kernel<T, 0>), grid, block, 0, st, w, row_bytes, K, e, out);
         err = hipGetLastError();
     });

@@ -67,3 +67,21 @@ def test_a8(bits, k, m, n):
     acc = q.double() @ qlin.w4a8_int8_grid(packed, s_rel, None, 64).double().T
     want = ((acc.float() * sx) * s_ch + bias).half()
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("qtype,k", [("Q8_0", 8224), ("Q8_0", 16384), ("Q6_K", 8448), ("Q6_K", 16640)])
+def test_wide_rows_decoded(qtype, k):
+    """Rows on both sides of the limits of the decode that keeps a row in registers (8192, 16384)."""
+    import qlin
+    n, m, ts, qk = 520, 1100, *{"Q8_0": (34, 32), "Q6_K": (210, 256)}[qtype]
+    raw = _ints((n, k // qk, ts), 0, 255, k).to(torch.uint8)
+    d = torch.full((n, k // qk, 1), 2.0 ** -7, dtype=torch.float16, device=DEV).view(torch.uint8)
+    if qtype == "Q8_0":
+        raw[:, :, :2] = d
+    else:
+        raw[:, :, 208:] = d
+        raw[:, :, 192:208] = _ints((n, k // qk, 16), 1, 4, 5).to(torch.uint8)
+    raw = raw.reshape(n, -1).contiguous()
+    x = _ints((m, k), -8, 8, k).half()
+    w = qlin.dequantize_gguf(raw, qtype, (n, k))  # at most 8 significant bits: exact in fp16
+    _check(qlin.gguf_linear(x, raw, qtype, (n, k), out_dtype=torch.float32), x, w)
