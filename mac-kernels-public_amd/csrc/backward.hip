@@ -13,6 +13,8 @@
 //     of n, k contiguous) and each MFMA fragment (8 consecutive n of one column) is one
 //     transposing 8-byte LDS read, widened in registers; the epilogue scales rows by 2^E[m],
 //     applies H to each 16-lane run of the row and rounds once to dx's dtype.
+#include <type_traits>
+
 #include "qlin_internal.h"
 #include "hadamard.h"
 
@@ -21,13 +23,10 @@ namespace qlin {
 namespace {
 
 constexpr int BW_BM = 128, BW_BK = 256, BW_BN = 64;
-constexpr int BW_RING = 2;  // register sets: a stage's loads are issued two stages before its use
-constexpr int BW_LS = BW_BN + 8;  // a tile LDS row stride in halves: 80 bytes, conflict-free fragment reads
 // weight tile in LDS as stored, [64 n][256 k] int8, row r's 16-byte chunk c at chunk c ^ 2 (r % 8):
-// the 16-byte writes of a row and the transposing fragment reads (8 rows x 2 chunk halves per
-// 16 lanes, even and odd chunks in the two groups of a 32-lane half) fall on distinct banks
-constexpr int BW_LB = BW_BK;
-constexpr int BW_BUF = BW_BM * BW_LS * 2 + BW_BN * BW_LB;  // bytes per pipeline buffer
+// the transposing fragment reads (8 rows x 2 chunk halves per 16 lanes, even and odd chunks in the two
+// groups of a 32-lane half) fall on distinct banks
+constexpr int BW_ASZ = BW_BM * BW_BN * 2, BW_BUF = BW_ASZ + BW_BN * BW_BK;  // bytes of a stage: a tile, weight tile
 __device__ __forceinline__ int bw_chunk(int row, int c) { return c ^ (2 * (row & 7)); }
 constexpr int BW_OW = BW_BK + BW_BK / 4;  // epilogue row stride in floats: 4 pad floats per 16
 
@@ -127,61 +126,95 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(uint32_t w0, uint32_t w1) {
     return f16x8{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
 }
 
-struct BwdRegs {
-    u32x4 a[2];  // 16 halves of one row of the a tile
-    u32x4 b[2];  // 16 int8 of each of two weight rows
-};
-
 typedef int v2i __attribute__((ext_vector_type(2)));
 
-// dx tile: rows m0 .. m0 + 127, columns k0 .. k0 + 255.  8 waves: wave w owns rows 64 (w / 4) ..
-// + 63 and columns 64 (w % 4) .. + 63 of the tile (2 x 2 sub-tiles of 32 x 32).  Stage = 64 values
-// of n: a tile [128][64] fp16 and weight tile [64][256] int8, the latter stored in LDS as read and
-// transposed by the fragment reads, then widened to fp16.  Two LDS buffers and two
-// register sets: each stage's global loads are issued two stages before it is computed.  WPE = 4
-// caps the registers at 128 so that two workgroups share a CU (grids beyond one round).  Measured
-// at M = 1056: a three-set ring, buffer loads with scalar row offsets and LDS DMA of both tiles in
-// three stages were slower.
-// The tile size sets the operand bytes per MFMA: at 128 x 256 a 64-value stage brings 32 KB for
-// 4.2 MFLOP.
-template <int G, int WPE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void bwd_gemm_kernel(BwdGemmArgs p) {
-    constexpr int SMEM = 2 * BW_BUF > 32 * BW_OW * 4 ? 2 * BW_BUF : 32 * BW_OW * 4;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// dx tile: rows m0 .. m0 + 127, columns k0 .. k0 + 255.  Wave w = 4 wm + wk owns rows 64 wm .. + 63 and
+// columns 64 wk .. + 63 of the tile (2 x 2 sub-tiles of 32 x 32).  A stage is 64 values of n: a tile
+// [128][64] fp16 and weight tile [64][256] int8, both brought in by LDS DMA as they lie in memory; the
+// weight fragments (8 consecutive n of one column) are transposing LDS reads, widened to fp16 in registers.
+//
+// The two groups of four waves take turns on the matrix cores, as in gemm_pp.h: stage t is a memory phase
+// (reads of the a fragments of stage t and the raw weights of stage t + 1, the requests of stage t + 3's
+// a tile and stage t + 4's weight tile) and a compute phase (16 MFMAs, stage t + 1's weights widened
+// between them), each ended by a barrier, and waves 4 .. 7 run one phase behind waves 0 .. 3, with which they share
+// their SIMDs.  LDS holds four stages.  With the memory phase of stage t of waves 0 .. 3 as phase 2t:
+//   the a tile of stage t is last read in phase 2t + 1 (waves 4 .. 7), the weight tile of stage t in phase
+//   2t - 1; their buffers are refilled from phase 2t + 2 and 2t on: in stage t + 1 and stage t;
+//   a wave's requests of stage t - 2 (a tile t + 1, weight tile t + 2) have landed before the barrier that
+//   ends its memory phase t: 8 younger ones may be outstanding.  Their first reads are in phase 2t + 2.
+// Against the same tile through registers with all waves in phase (matrix cores about a third busy), M1056
+// K6144 N16384: 311 -> 214 us, 992 TFLOP/s; 216 of 256 CUs have a tile there and 8% of the tile rows are padding.
+template <int G>
+__global__ __launch_bounds__(512) void bwd_gemm_kernel(BwdGemmArgs p) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[4 * BW_BUF];
+    static_assert(32 * BW_OW * 4 <= 4 * BW_BUF, "output staging must fit");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r32 = lane & 31, h = lane >> 5, wm = wave >> 2, wk = wave & 3;
     const int64_t m0 = (int64_t)blockIdx.y * BW_BM, k0 = (int64_t)blockIdx.x * BW_BK;
-    // global load assignment: a row tid / 4, 16 halves at 16 (tid % 4); weight rows tid / 16 and
-    // 32 + tid / 16 of the stage, 16 bytes at column 16 (tid % 16) of the tile
-    const f16* ap = p.a + min(m0 + tid / 4, p.M - 1) * p.lda + 16 * (tid & 3);
-    const int brow = tid >> 4, bc = tid & 15;
-    const int8_t* bp = p.b + min(k0 + 16 * bc, p.K - 16);  // columns past K re-read (never stored)
-    const int nst = (int)(p.lda / BW_BN);  // lda is N rounded up to 128; a is zero past N
-    auto load = [&](int s, BwdRegs& r) {
-        const u32x4* pa = reinterpret_cast<const u32x4*>(ap + (int64_t)BW_BN * s);
-        r.a[0] = pa[0];
-        r.a[1] = pa[1];
+    const int nst = (int)(p.lda / BW_BN);  // lda is N rounded up to 128: even; a is zero past N
+    // DMA instruction i of a tile fills its 16-byte chunks u = 512 i + tid: a tile row u / 8, logical chunk
+    // (u % 8) ^ (row / 2) % 8; weight row u / 16, logical chunk bw_chunk(row, u % 16)
+    const f16* asrc[2];
+    const int8_t* bsrc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int u = 512 * i + tid, ar = u / 8, br = u / 16;
+        asrc[i] = p.a + min(m0 + ar, p.M - 1) * p.lda + 8 * ((u % 8) ^ ((ar / 2) % 8));
+        // columns past K re-read (never stored)
+        bsrc[i] = p.b + min<int64_t>(br, p.N - 1) * p.ldb + min(k0 + 16 * bw_chunk(br, u % 16), p.K - 16);
+    }
+    auto dma_a = [&](int t, int buf) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            lds_dma16(asrc[i] + (int64_t)BW_BN * min(t, nst - 1), smem + buf * BW_BUF + 16 * (512 * i + 64 * wave));
+    };
+    // called for t = 0, 1, ..: a row's pointer moves on while the next row is one of the weight's, and stays
+    // from then on (rows past N meet a = 0)
+    auto dma_b = [&](int t, int buf) {
+        const int64_t left = p.N - (int64_t)BW_BN * (t + 1);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int64_t n = min((int64_t)BW_BN * s + 32 * i + brow, p.N - 1);  // rows past N meet a = 0
-            r.b[i] = *reinterpret_cast<const u32x4*>(bp + n * p.ldb);
+            lds_dma16(bsrc[i], smem + buf * BW_BUF + BW_ASZ + 16 * (512 * i + 64 * wave));
+            bsrc[i] += 32 * i + tid / 16 < left ? BW_BN * p.ldb : 0;
         }
     };
-    auto store = [&](const BwdRegs& r, int buf) {
-        f16* As = reinterpret_cast<f16*>(smem + buf * BW_BUF);
-        uint8_t* Bs = smem + buf * BW_BUF + BW_BM * BW_LS * 2;
-        f16* ad = As + (tid >> 2) * BW_LS + 16 * (tid & 3);
-        *reinterpret_cast<u32x4*>(ad) = r.a[0];
-        *reinterpret_cast<u32x4*>(ad + 8) = r.a[1];
+    // a fragments of stage t; raw weights of stage t + 1; widened weights of even and odd stages
+    f16x8 af[2][4], bf[2][2][4];
+    v2i raw[2][4];
+    auto read_a = [&](int buf) {
+        const uint8_t* src = smem + buf * BW_BUF + (64 * wm + r32) * 128;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int row = 32 * i + brow;
-            *reinterpret_cast<u32x4*>(Bs + row * BW_LB + 16 * bw_chunk(row, bc)) = r.b[i];
-        }
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                af[i][st] = *reinterpret_cast<const f16x8*>(src + 4096 * i + 16 * ((2 * st + h) ^ ((r32 / 2) % 8)));
     };
     // transposing fragment reads: in each 16-lane group, lane i names row nb + i / 2 at column
-    // kc + 8 (i % 2) and receives column kc + i of rows nb .. nb + 7 (ds_read_b64_tr_b8)
-    const int gi = lane & 15, g = lane >> 4;
+    // kc + 8 (i % 2) and receives column kc + i of rows nb .. nb + 7.  As one asm block that waits for
+    // them: ahead of the builtin the compiler waits for every DMA in flight.
+    const int gi = lane & 15, g = lane >> 4, brow = 8 * (g >> 1) + (gi >> 1);
+    uint32_t bad[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        bad[j] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem + BW_ASZ + brow * BW_BK +
+                 16 * bw_chunk(brow, (64 * wk + 32 * j + 16 * (g & 1)) >> 4) + 8 * (gi & 1);
+    auto read_b = [&](int buf) {
+        asm volatile(
+            "ds_read_b64_tr_b8 %0, %8\n"
+            "ds_read_b64_tr_b8 %1, %9\n"
+            "ds_read_b64_tr_b8 %2, %8 offset:4096\n"
+            "ds_read_b64_tr_b8 %3, %9 offset:4096\n"
+            "ds_read_b64_tr_b8 %4, %8 offset:8192\n"
+            "ds_read_b64_tr_b8 %5, %9 offset:8192\n"
+            "ds_read_b64_tr_b8 %6, %8 offset:12288\n"
+            "ds_read_b64_tr_b8 %7, %9 offset:12288\n"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(raw[0][0]), "=&v"(raw[1][0]), "=&v"(raw[0][1]), "=&v"(raw[1][1]), "=&v"(raw[0][2]),
+              "=&v"(raw[1][2]), "=&v"(raw[0][3]), "=&v"(raw[1][3])
+            : "v"(bad[0] + buf * BW_BUF), "v"(bad[1] + buf * BW_BUF)
+            : "memory");
+    };
+    auto widen = [&](int j, int st) { return i8x8_to_f16((uint32_t)raw[j][st].x, (uint32_t)raw[j][st].y); };
     f32x16 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -189,46 +222,75 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    auto compute = [&](int buf) {
-        const f16* As = reinterpret_cast<const f16*>(smem + buf * BW_BUF);
-        const uint8_t* Bs = smem + buf * BW_BUF + BW_BM * BW_LS * 2;
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stage = [&](int t, auto q) {
+        constexpr int Q = decltype(q)::value;  // t % 4
+        read_a(Q);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b((Q + 1) % 4);
+        __builtin_amdgcn_sched_barrier(0);
+        dma_a(t + 3, (Q + 3) % 4);
+        dma_b(t + 4, Q);
+        wait_lgkmcnt0();
+        wait_vmcnt<8>();
+        barrier();
 #pragma unroll
-        for (int st = 0; st < BW_BN / 16; ++st) {
-            f16x8 af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                af[i] = *reinterpret_cast<const f16x8*>(As + (64 * wm + 32 * i + r32) * BW_LS + 16 * st + 8 * h);
+        for (int st = 0; st < 4; ++st)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int row = 16 * st + 8 * (g >> 1) + (gi >> 1), kc = 64 * wk + 32 * j + 16 * (g & 1);
-                const uint8_t* src = Bs + row * BW_LB + 16 * bw_chunk(row, kc >> 4) + 8 * (gi & 1);
-                const v2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)src);
-                bf[j] = i8x8_to_f16((uint32_t)w.x, (uint32_t)w.y);
+                bf[(Q + 1) % 2][j][st] = widen(j, st);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][st], bf[Q % 2][j][st], acc[i][j], 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < 16; ++i) {  // an MFMA, then five of the 80 widening operations
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
         }
+        barrier();
     };
-    // stage s lives in register set s % 2 and LDS buffer s % 2.  Loads past the last stage re-read
-    // stage nst - 1 (in bounds) and are never computed.
-    BwdRegs r0, r1;
-    load(0, r0);
-    load(1, r1);
-    store(r0, 0);
-    __syncthreads();
-    const int last = nst - 1;
-    for (int s = 0; s < nst; s += BW_RING) {
-        load(min(s + 2, last), r0);
-        compute(0);
-        store(r1, 1);
-        __syncthreads();
-        load(min(s + 3, last), r1);
-        compute(1);
-        store(r0, 0);
-        __syncthreads();
+    // the requests of stages -4 .. -1, in their order
+    dma_b(0, 0);
+    dma_a(0, 0);
+    dma_b(1, 1);
+    dma_a(1, 1);
+    dma_b(2, 2);
+    dma_a(2, 2);
+    dma_b(3, 3);
+    wait_vmcnt<8>();  // weight tiles 0 and 1, a tile 0
+    barrier();
+    read_b(0);
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bf[0][j][st] = widen(j, st);
+    barrier();
+    if (wm) barrier();  // waves 4 .. 7: one phase behind
+    constexpr std::integral_constant<int, 0> q0{};
+    constexpr std::integral_constant<int, 1> q1{};
+    constexpr std::integral_constant<int, 2> q2{};
+    constexpr std::integral_constant<int, 3> q3{};
+    int t = 0;
+    for (; t + 3 < nst; t += 4) {
+        stage(t, q0);
+        stage(t + 1, q1);
+        stage(t + 2, q2);
+        stage(t + 3, q3);
     }
+    if (t < nst) {
+        stage(t, q0);
+        stage(t + 1, q1);
+    }
+    if (!wm) barrier();
+    wait_vmcnt<0>();
+    __syncthreads();  // every wave is past the main loop, its DMAs included
     // epilogue, four passes of 32 rows through LDS (the pipeline buffers are no longer read):
     // element (row, c) at row * BW_OW + c + 4 (c / 16)
     float* ot = reinterpret_cast<float*>(smem);
@@ -277,7 +339,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
 hipError_t run_bwd_rows(const void* dy, int dy_dt, int64_t ldd, int64_t M, int64_t N, const void* s, int s_dt,
                         int64_t s_stride, f16* a, int64_t lda, int32_t* e, hipStream_t st) {
     if (M == 0) return hipSuccess;
-    if (lda < N || lda % (BW_RING * BW_BN)) return hipErrorInvalidValue;
+    if (lda < N || lda % (2 * BW_BN)) return hipErrorInvalidValue;
     bool ok = false;
     auto go = [&](auto dy_tag, auto s_tag) {
         using T = decltype(dy_tag);
@@ -302,18 +364,13 @@ hipError_t run_bwd_gemm(const BwdGemmArgs& p, hipStream_t st) {
     if (p.M == 0 || p.K == 0) return hipSuccess;
     // the kernel's loads assume: K a multiple of 16 (4-byte weight loads from clamped columns),
     // 16-byte aligned weight rows, lda a multiple of 128 covering N, N >= 1
-    if (p.K % 16 || p.ldb % 16 || (uintptr_t)p.b % 16 || p.lda % (BW_RING * BW_BN) || p.lda < p.N || p.N < 1 ||
+    if (p.K % 16 || p.ldb % 16 || (uintptr_t)p.b % 16 || p.lda % (2 * BW_BN) || p.lda < p.N || p.N < 1 ||
         (uintptr_t)p.a % 16)
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)((p.K + BW_BK - 1) / BW_BK), (unsigned)((p.M + BW_BM - 1) / BW_BM));
     bool ok = false;
-    // grids of more than one workgroup per CU: 128 registers (4 waves per SIMD, a few spilled), two
-    // workgroups per CU (mlp.down-sized grids: 300 against 319 us); one round: the unconstrained
-    // kernel (148 against 154 us)
-    const bool two = (int64_t)grid.x * grid.y > 256;
     auto go = [&]<int G>() {
-        if (two) hipLaunchKernelGGL((bwd_gemm_kernel<G, 4>), grid, dim3(512), 0, st, p);
-        else hipLaunchKernelGGL((bwd_gemm_kernel<G, 1>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((bwd_gemm_kernel<G>), grid, dim3(512), 0, st, p);
         ok = true;
     };
     if (!dispatch_group(p.G, go) || !ok) return hipErrorInvalidValue;

@@ -69,6 +69,16 @@ def test_a8(bits, k, m, n):
     assert torch.equal(y, want)
 
 
+@pytest.mark.parametrize("m,k", [(1, 16), (129, 528)])  # columns and rows of a tile past the matrix
+@pytest.mark.parametrize("n", [1, 63, 65, 129, 256, 300, 513, 900])  # 2 to 16 stages of 64, the last of them ragged
+def test_grad_input(n, m, k):
+    import qlin
+    dy = _ints((m, n), -8, 8, n).half()
+    q = _ints((n, k), -128, 127, m).to(torch.int8)
+    dx = qlin.int8_linear_grad_input(dy, q, torch.full((n,), 0.5, device=DEV), False, 256, out_dtype=torch.float32)
+    _check(dx, dy, q.float().T / 2)
+
+
 @pytest.mark.parametrize("qtype,k", [("Q8_0", 8224), ("Q8_0", 16384), ("Q6_K", 8448), ("Q6_K", 16640)])
 def test_wide_rows_decoded(qtype, k):
     """Rows on both sides of the limits of the decode that keeps a row in registers (8192, 16384)."""
