@@ -1158,6 +1158,12 @@ hipError_t launch1(const GemmF16Args& a, hipStream_t st) {
                 auto tiles_of = [](const GemmF16Args& g, int bm) { return ((g.M + bm - 1) / bm) * ((g.N + 255) / 256); };
                 const hipError_t err = launch_wo256(dim3((unsigned)tiles_of(top, 256)), top, st);
                 if (err != hipSuccess) return err;
+                // a rest of so few rows that the ring kernel's tiles below run in one round: its workgroups share
+                // the weights out over more CUs, and few tile rows are padding (M1056 K6144 N16384, the last 32
+                // rows: 27.5 against 90 us; whole calls, 1152 rows 269 -> 212 us, M2240 K3072 N8192 151 -> 121,
+                // M3648 K5120 N4608 235 -> 168)
+                if ((rest.M + 63) / 64 * ((a.N + 127) / 128) <= 256 && (rest.M + 127) / 128 * ((a.N + 127) / 128) < 160)
+                    return launch1<WO_INT8, 0>(rest, st);
                 hipLaunchKernelGGL((gemm_wo_dma_kernel<128, 3>), dim3((unsigned)tiles_of(rest, 128)), dim3(512), 0, st, rest);
                 return hipGetLastError();
             }
