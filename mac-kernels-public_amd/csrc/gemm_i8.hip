@@ -1041,8 +1041,9 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_i8dma_kernel(GemmI8Args p
 }
 
 // 256 x 256 tiles over the decoded int8 grid: the main loop of gemm_pp.h, then the epilogue of
-// gemm_i8dma_kernel, in passes of 64 rows.  us of this kernel against the 32 x 32 loop with one barrier a
-// k-tile that it replaces: PPTIMES
+// gemm_i8dma_kernel, in passes of 64 rows.  Against the 32 x 32 loop with one
+// barrier a k-tile that it replaces: W6A8 MLP 5120 -> 13824 -> 5120 at 9504 rows, both calls whole, 1542 -> 1412 us;
+// W4A8 M4096 K3072 N12288 190 us with either (24 k-tiles: prologue and epilogue weigh more).
 template <int LDU = -1>
 __global__ __launch_bounds__(512) void gemm_i8pp_kernel(GemmI8Args p, const int8_t* __restrict__ w8) {
     constexpr int NT = 512, BT = 256;
