@@ -95,3 +95,21 @@ def test_wide_rows_decoded(qtype, k):
     x = _ints((m, k), -8, 8, k).half()
     w = qlin.dequantize_gguf(raw, qtype, (n, k))  # at most 8 significant bits: exact in fp16
     _check(qlin.gguf_linear(x, raw, qtype, (n, k), out_dtype=torch.float32), x, w)
+
+
+@pytest.mark.parametrize("m,n", [(1025, 16384), (1090, 16300), (2100, 8100)])  # rests of 1, 66 and 52 rows: 32- and 64-row tiles
+@pytest.mark.parametrize("k", [64, 384, 512])
+def test_int8_rest(k, m, n):
+    """Whole rounds of 256 x 256 tiles, then the last rows through the ring kernel."""
+    import qlin
+    x = _ints((m, k), -8, 8, k).half()
+    q = _ints((n, k), -128, 127, m).to(torch.int8)
+    r = _ints((m, n), -4, 4, 7).float()
+    s = torch.full((n,), 0.5, device=DEV)
+    _check(qlin.int8_linear(x, q, s, out_dtype=torch.float32), x, q.float() / 2)
+    _check(qlin.int8_linear(x, q, s, out_dtype=torch.float32, residual=r), x, q.float() / 2, r.double())
+
+
+@pytest.mark.parametrize("m", [2049, 2148, 2305, 2500])  # rests of 1, 100, 257 and 452 rows: 64, 64, 128 and 128 columns
+def test_a8_rest(m):
+    test_a8(4, 256, m, 8192)
