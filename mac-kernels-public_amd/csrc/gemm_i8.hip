@@ -1326,6 +1326,11 @@ hipError_t launch_o(const GemmI8Args& p, hipStream_t st) {
             }
         };
         if (ldu != -1 && ldu != DT_BF16 && ldu != DT_F16 && ldu != DT_F32) return hipErrorInvalidValue;
+        // the two-group loop from K = 3584: its first loads and its 128 KiB per workgroup are not overlapped with
+        // another tile's work, and short rows do not win that back (us, without and with it: M9504 K1024 N16384 262,
+        // 312; M7000 K1536 N12288 197, 217; M8192 K2048 N16384 336, 349; M4608 K3072 N9216 167, 168; M4096 K4096
+        // N8192 157, 153; M2500 K5120 N13824 241, 219; M1500 K16384 N8192 259, 222)
+        const bool pp = p.K >= 3584;
         const int64_t m1 = ldu == -1 && tiles(256, 256) >= 192 ? tail_split_rows(p.M, p.N) : 0;
         if (m1) {  // whole rounds of 256 x 256 tiles, then the rest as one round of 128 x 256 tiles
             GemmI8Args top = p, rest = p;
@@ -1336,7 +1341,8 @@ hipError_t launch_o(const GemmI8Args& p, hipStream_t st) {
             rest.y = (uint8_t*)p.y + m1 * p.ldy * dt_bytes(p.y_dtype);
             if (p.res.r) rest.res.r = (const uint8_t*)p.res.r + m1 * p.res.ldr * dt_bytes(p.res.r_dt);
             auto tiles_of = [](const GemmI8Args& g, int bm) { return ((g.M + bm - 1) / bm) * ((g.N + 255) / 256); };
-            hipLaunchKernelGGL(gemm_i8pp_kernel<>, dim3((unsigned)tiles_of(top, 256)), dim3(512), 0, st, top, top.w8);
+            if (pp) hipLaunchKernelGGL(gemm_i8pp_kernel<>, dim3((unsigned)tiles_of(top, 256)), dim3(512), 0, st, top, top.w8);
+            else hipLaunchKernelGGL((gemm_i8dma_kernel<256, 256, 128, 2, false>), dim3((unsigned)tiles_of(top, 256)), dim3(512), 0, st, top, top.w8);
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) return err;
             // the narrowest tiles that still run in one round: a rest of few rows is bound by how many CUs share
@@ -1350,7 +1356,9 @@ hipError_t launch_o(const GemmI8Args& p, hipStream_t st) {
                 hipLaunchKernelGGL((gemm_i8dma_kernel<128, 256, 128, 2, false>), dim3((unsigned)rest_tiles(256)), dim3(512), 0, st, rest, rest.w8);
             return hipGetLastError();
         }
-        if (tiles(256, 256) >= 192) {
+        if (tiles(256, 256) >= 192 && !pp) {
+            go.template operator()<256, 256>();
+        } else if (tiles(256, 256) >= 192) {
             const dim3 grid((unsigned)tiles(256, 256));
             switch (ldu) {
                 case -1: hipLaunchKernelGGL(gemm_i8pp_kernel<>, grid, dim3(512), 0, st, p, p.w8); break;
