@@ -533,7 +533,7 @@ hipError_t launch(const GgufGemvArgs& a, hipStream_t st) {
 // the weight stream, the decode's VALU (Q4_K: 5 operations per two weights) and, at a few MB, by the
 // latency of the first bytes.  In a HIP graph over cold weights, us against the kernels that these
 // rows took before (the small-M one, or the prologue and the kernel below): Q4_K K5120 N13824 bf16
-// 13.7 against 30.8 (2.9 TB/s), Q6_K K13824 N5120 bf16 22.0 against 45.2, IQ4_XS K14336 N4096 bf16
+// 13.0 against 30.8 (3.1 TB/s), Q6_K K13824 N5120 bf16 19.9 against 45.2, IQ4_XS K14336 N4096 bf16
 // 12.8 against 23.4, Q8_0 K11264 N4096 bf16 11.9 against 20.8, Q4_K K = N = 4096 bf16 5.4 against
 // 7.5.  fp16 rows keep the kernel below at its K (Q4_K 5.0, Q6_K 5.6, Q8_0 5.6 us there).
 //
@@ -698,7 +698,6 @@ struct GVRow<gguf::IQ4_XS> {
     }
 };
 
-constexpr int GVR_THREADS = 256;
 constexpr int GVR_MAX_K = 16384;  // 32 KiB of operand in LDS
 
 // 8 raw activations as loaded (held until the weight loads are out)
@@ -714,14 +713,14 @@ template <typename TX> struct RawUnit {
     }
 };
 
-template <int T, int LPR, typename TX>
-__global__ __launch_bounds__(GVR_THREADS) void gguf_gemv_rows_kernel(const TX* x, const int32_t* xexp, const uint8_t* w,
+template <int T, int LPR, typename TX, int NT>
+__global__ __launch_bounds__(NT) void gguf_gemv_rows_kernel(const TX* x, const int32_t* xexp, const uint8_t* w,
                                                             int64_t row_bytes, int N, int K, const void* bias,
                                                             int bias_dt, void* y, int y_dt) {
     using F = GV<T>;
     constexpr bool RAW = !std::is_same<TX, f16>::value;  // fp16 rows are used as they are
     constexpr bool TAB = F::LUT;
-    constexpr int NT = GVR_THREADS, NW = NT / 64, NX = GVR_MAX_K / 8 / NT;
+    constexpr int NW = NT / 64, NX = GVR_MAX_K / 8 / NT;
     constexpr int VC = F::VC, RPW = 64 / LPR;
     constexpr bool MIN = T == gguf::Q4_K || T == gguf::Q5_K;  // block minima: sums of x per 32 values
     __shared__ __attribute__((aligned(16))) u32x4 xop[GVR_MAX_K / 8];
@@ -859,18 +858,21 @@ __global__ __launch_bounds__(GVR_THREADS) void gguf_gemv_rows_kernel(const TX* x
     if (steps & 1) step(r0);
 }
 
-// Lanes per row L and row groups per wave G.  The fastest grids measured have at most 1024 waves (a
-// workgroup of 4 per CU: with more than one workgroup on some CUs they wait for those, and each
-// redoes the operand); of those, the shortest wave: G row groups of IT chunks and one reduction
-// each.  us for each L at its best G, the one taken first (before the codes were made exact): Q4_K
-// K5120 N13824 L8 11.2, L16 12.3, L32 14.7; Q6_K K13824 N5120 L8 23.0, L16 22.1, L32 22.1; Q8_0 K11264
-// N4096 L16 11.9, L64 11.2; Q4_K K3072 N3072 L16 4.6, L32 5.0, L8 5.4; Q4_K K8192 N1024 L64 4.4, L32 5.0.
-inline int gemv_rows_lanes(int N, int C, int& G) {
+// Lanes per row L and row groups per wave G.  The fastest grids measured have at most one workgroup per
+// CU (with more on some CUs they wait for those, and each redoes the operand): W = 1024 waves in
+// workgroups of 4, 2048 in workgroups of 8.  Of those, the shortest wave: G row groups of IT chunks and
+// one reduction each; of equally short ones the most lanes per row, whose loads read longer pieces of
+// fewer rows and which keep more waves in flight.  us for each L at its best G: Q6_K K13824 N5120 L8
+// 25.0, L16 23.7, L32 21.0, L64 19.9 (L8, L32 and L64 are equally short); Q4_K there L8 17.8, L64 15.9;
+// Q8_0 K6912 N5120 L8 13.2, L64 10.8.  Q4_K K5120 N13824 L8 14.0, L16 16.6, L32 19.0; Q4_K K3072 N3072
+// L16 5.3, L32 5.6, L8 6.1; Q4_K K8192 N1024 L64 4.8, L32 5.6.
+inline int gemv_rows_lanes(int N, int C, int W, int& G) {
     int best = 0, L = 8;
     for (int l : {8, 16, 32, 64}) {
+        if (l > 8 && l / 2 >= C) break;  // half the lanes would have no chunk
         const int64_t waves = ((int64_t)N * l + 63) / 64;
-        const int g = (int)((waves + 1023) / 1024), cost = g * ((C + l - 1) / l + 1);
-        if (!best || cost < best) {
+        const int g = (int)((waves + W - 1) / W), cost = g * ((C + l - 1) / l + 1);
+        if (!best || cost <= best) {
             best = cost;
             L = l;
             G = g;
@@ -879,14 +881,14 @@ inline int gemv_rows_lanes(int N, int C, int& G) {
     return L;
 }
 
-template <int T, typename TX>
-hipError_t launch_rows(const GgufGemvArgs& a, hipStream_t st) {
+template <int T, typename TX, int NT>
+hipError_t launch_rows_nt(const GgufGemvArgs& a, hipStream_t st) {
     int G = 1;
-    const int L = gemv_rows_lanes(a.N, a.K / GV<T>::VC, G);
-    const int64_t rows = (int64_t)GVR_THREADS / L * G;
-    const dim3 grid((unsigned)((a.N + rows - 1) / rows)), block(GVR_THREADS);
+    const int L = gemv_rows_lanes(a.N, a.K / GV<T>::VC, 4 * NT, G);
+    const int64_t rows = (int64_t)NT / L * G;
+    const dim3 grid((unsigned)((a.N + rows - 1) / rows)), block(NT);
 #define QLIN_GVR(LV)                                                                                                   \
-    hipLaunchKernelGGL((gguf_gemv_rows_kernel<T, LV, TX>), grid, block, 0, st, (const TX*)a.x, a.xexp, a.w, a.row_bytes, \
+    hipLaunchKernelGGL((gguf_gemv_rows_kernel<T, LV, TX, NT>), grid, block, 0, st, (const TX*)a.x, a.xexp, a.w, a.row_bytes, \
                        a.N, a.K, a.bias, a.bias_dtype, a.y, a.y_dtype)
     switch (L) {
         case 8: QLIN_GVR(8); break;
@@ -896,6 +898,18 @@ hipError_t launch_rows(const GgufGemvArgs& a, hipStream_t st) {
     }
 #undef QLIN_GVR
     return hipGetLastError();
+}
+
+// Workgroups of 8 waves (twice the loads in flight per operand) for large Q4_K tensors: K5120 N13824 14.3
+// -> 13.0 us, K13824 N5120 16.4 -> 15.2, K4096 N14336 11.7 -> 11.2, K16384 N8192 21.5 -> 20.4; below 50
+// million weights the longer start loses (K5120 N8192 8.6 against 10.0), and the other types are
+// limited by their decode (Q5_K K3584 N18944 16.9 against 17.3, Q6_K K13824 N5120 19.9 against 21.1).
+template <int T, typename TX>
+hipError_t launch_rows(const GgufGemvArgs& a, hipStream_t st) {
+    if constexpr (T == gguf::Q4_K) {
+        if ((int64_t)a.N * a.K >= 50000000) return launch_rows_nt<T, TX, 512>(a, st);
+    }
+    return launch_rows_nt<T, TX, 256>(a, st);
 }
 
 template <typename Fn>
