@@ -51,7 +51,7 @@ def test_int8(k, m, n):
 
 
 @pytest.mark.parametrize("m,n", [(3585, 3500), (600, 16400)])  # 210 and 195 tiles
-@pytest.mark.parametrize("bits,k", [(4, 128), (6, 256), (4, 384), (6, 640)])
+@pytest.mark.parametrize("bits,k", [(4, 128), (6, 256), (4, 384), (6, 640), (4, 3584), (6, 3712)])  # two groups from 3584
 def test_a8(bits, k, m, n):
     import qlin
     from qlin.quantize import pack_codes
@@ -113,3 +113,4 @@ def test_int8_rest(k, m, n):
 @pytest.mark.parametrize("m", [2049, 2148, 2305, 2500])  # rests of 1, 100, 257 and 452 rows: 64, 64, 128 and 128 columns
 def test_a8_rest(m):
     test_a8(4, 256, m, 8192)
+    test_a8(4, 3584, m, 8192)
