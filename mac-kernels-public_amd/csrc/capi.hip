@@ -275,6 +275,13 @@ float* lora_t_final(float* t, int64_t M, int64_t K, int64_t R) {
     return S > 1 ? t + (int64_t)S * M * R : t;
 }
 
+// A linear over no values (K = 0): its output is the bias.  The kernels below clamp their loads to a row's last
+// values, so none of them is launched without any.
+qlin_status no_values(const qlin_tensor* bias, int bias_dtype, const Mat& Y, hipStream_t st) {
+    return hip_status(run_bias_rows(bias ? bias->data : nullptr, bias_dtype, Y.data, Y.dtype, Y.ld, Y.rows, Y.cols, st),
+                      "bias rows");
+}
+
 // Runs the weight-only prologue unless x is already usable as the fp16 MFMA operand (fp16, no
 // rotation, aligned rows), in which case x itself is used and no exponents are needed.
 qlin_status wo_activations(const Mat& X, int G, Carver& ws, hipStream_t st, const f16*& xo, int64_t& ldx,
@@ -613,6 +620,7 @@ static qlin_status int8_linear_impl(const qlin_tensor* x, const qlin_tensor* qda
     if (workspace_bytes < need) return fail(QLIN_EWORKSPACE, "workspace %zu < %zu", workspace_bytes, need);
     if (M == 0 || N == 0) return QLIN_OK;
     hipStream_t st = (hipStream_t)stream;
+    if (K == 0 && !L) return R ? QLIN_NOT_FUSED : no_values(bias, bdt, Y, st);
     Carver ws{(uint8_t*)workspace, workspace_bytes};
     if (R) {
         // only the large-M GEMM applies a residual: its operands as run_gemm_f16 will see them
@@ -645,6 +653,7 @@ static qlin_status int8_linear_impl(const qlin_tensor* x, const qlin_tensor* qda
         if (M <= INT8_SMALLM_MAX_M || !gemm_f16_fuses_lora(a))
             return fail(QLIN_EUNSUPPORTED, "the LoRA term is fused only into the large-M GEMM (rank a multiple of 8, "
                                            "16-byte aligned lora_up rows)");
+        if (K == 0) return no_values(bias, bdt, Y, st);
         const float* tf = nullptr;
         if ((s = hip_status(run_lora_t(lora_down_args(X, D, t), st, &tf), "lora down"))) return s;
         if ((s = wo_activations(X, convrot_groupsize, ws, st, a.x, a.ldx, a.xexp))) return s;
@@ -782,6 +791,7 @@ static qlin_status gguf_linear_impl(const qlin_tensor* x, const void* weight, in
     if (M == 0 || N == 0) return QLIN_OK;
     const int64_t row_bytes = (K / qk) * ts;
     hipStream_t st = (hipStream_t)stream;
+    if (K == 0) return R ? QLIN_NOT_FUSED : no_values(bias, bdt, Y, st);
     Carver ws{(uint8_t*)workspace, workspace_bytes};
     const bool aligned = ((uintptr_t)weight % 4) == 0;
     // a residual rides in the epilogue of the split kernel (or its reduction) and of the GEMM over
@@ -1023,6 +1033,7 @@ static qlin_status w4a8_linear_impl(const qlin_tensor* x, const qlin_tensor* qda
     if (workspace_bytes < need) return fail(QLIN_EWORKSPACE, "workspace %zu < %zu", workspace_bytes, need);
     if (M == 0 || N == 0) return QLIN_OK;
     hipStream_t st = (hipStream_t)stream;
+    if (K == 0 && !L) return R ? QLIN_NOT_FUSED : no_values(bias, bdt, Y, st);
     Carver ws{(uint8_t*)workspace, workspace_bytes};
     // workspace: int8 activations, their scales, the decoded weight grid (a8_grid_in_workspace), then
     // LoRA's t
@@ -1051,6 +1062,7 @@ static qlin_status w4a8_linear_impl(const qlin_tensor* x, const qlin_tensor* qda
                                            "once (from 512 rows, or above 32 rows on grids of fewer than 192 tiles of 256 x "
                                            "256; a group size that is a multiple of 64), for a rank that is a multiple of 8 "
                                            "with 16-byte aligned lora_up rows");
+        if (K == 0) return no_values(bias, bdt, Y, st);
         const float* tf = nullptr;
         if ((s = hip_status(run_lora_t(lora_down_args(X, D, t), st, &tf), "lora down"))) return s;
     }

@@ -4,6 +4,7 @@
 // (roblennon/mac-kernels-public docs/upstream/comfy-kitchen-mps-backend.md:52;
 // tests/test_lora_sidepath.py:378-386), in fp32 with one rounding.
 // Eight outputs per thread, 16-byte loads and stores where rows allow them.
+// Also the linear over no values (K = 0), whose output is the bias.
 #include "qlin_internal.h"
 
 namespace qlin {
@@ -37,7 +38,24 @@ __global__ __launch_bounds__(256) void residual_kernel(ResidualArgs a) {
     store8_rt(a.y, a.y_dt, m * a.ldy + n, o, cnt, yvec);
 }
 
+__global__ __launch_bounds__(256) void bias_rows_kernel(const void* bias, int bias_dt, void* y, int y_dt, int64_t ldy,
+                                                        int64_t M, int64_t N) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= M * N) return;
+    const int64_t m = i / N, n = i % N;
+    store_rt(y, y_dt, m * ldy + n, bias ? load_rt(bias, bias_dt, n) : 0.0f);
+}
+
 }  // namespace
+
+hipError_t run_bias_rows(const void* bias, int bias_dt, void* y, int y_dt, int64_t ldy, int64_t M, int64_t N,
+                         hipStream_t st) {
+    if (M == 0 || N == 0) return hipSuccess;
+    if (y_dt != DT_F32 && y_dt != DT_F16 && y_dt != DT_BF16) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(bias_rows_kernel, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, bias, bias_dt, y, y_dt,
+                       ldy, M, N);
+    return hipGetLastError();
+}
 
 hipError_t run_residual(const ResidualArgs& a, hipStream_t st) {
     if (a.M == 0 || a.N == 0) return hipSuccess;

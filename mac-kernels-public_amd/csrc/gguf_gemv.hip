@@ -929,14 +929,16 @@ bool dispatch_gemv(int t, Fn&& f) {
 }  // namespace
 
 bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void* w, const void* x) {
-    // Q6_K rows of an odd number of blocks start 2 bytes off a dword, which its loads realign
-    if (K > GVR_MAX_K || (uintptr_t)w % 4 || (uintptr_t)x % 16 || row_bytes % (type == gguf::Q6_K ? 2 : 4)) return false;
+    // The kernel's loads are clamped to a row's last chunk, so a row has one: K = 0 is not taken.  Q6_K rows
+    // of an odd number of blocks start 2 bytes off a dword, which its loads realign.
+    if (K < 1 || K > GVR_MAX_K || (uintptr_t)w % 4 || (uintptr_t)x % 16 || row_bytes % (type == gguf::Q6_K ? 2 : 4)) return false;
     bool ok = false;
     dispatch_gemv(type, [&]<int T>() { ok = K % GV<T>::VC == 0; });
     return ok;
 }
 
 hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st) {
+    if (!gguf_gemv_rows_supported(a.type, a.K, a.row_bytes, a.w, a.x)) return hipErrorInvalidValue;
     if (a.y_dtype != DT_F32 && a.y_dtype != DT_F16 && a.y_dtype != DT_BF16) return hipErrorInvalidValue;
     hipError_t err = hipErrorInvalidValue;
     dispatch_gemv(a.type, [&]<int T>() {

@@ -181,7 +181,8 @@ struct GgufGemvArgs {
 };
 bool gguf_gemv_supported(int type, int64_t M, int64_t K, int64_t row_bytes, const void* w, const void* x);
 hipError_t run_gguf_gemv(const GgufGemvArgs& a, hipStream_t st);
-// The GEMV over rows of any whole number of chunks (64 values for Q8_0, else 128) up to 16384.
+// The GEMV over rows of any whole number of chunks (64 values for Q8_0, else 128) up to 16384, at
+// least one.
 bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void* w, const void* x);
 hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st);
 
@@ -408,6 +409,9 @@ struct ResidualArgs {
     int64_t M = 0, N = 0;
 };
 hipError_t run_residual(const ResidualArgs& a, hipStream_t st);
+// y[m, n] = bias[n] (0 without one): the linear over no values.
+hipError_t run_bias_rows(const void* bias, int bias_dt, void* y, int y_dt, int64_t ldy, int64_t M, int64_t N,
+                         hipStream_t st);
 
 // ---- frozen-weight input gradient (backward.hip) ----
 struct BwdGemmArgs {

@@ -279,3 +279,15 @@ def test_int8_convrot_quantizer_matches_oracle():
     q, s = quantize_int8_convrot_weight(w, 256)
     oq, os_ = O.quantize_int8_rowwise(O.rotate(w, 256))
     assert np.array_equal(q, oq) and np.array_equal(s, os_.reshape(-1))
+
+
+@pytest.mark.parametrize("ggml_type", [2, 8, 12, 13, 14, 20, 23])
+def test_one_row_gguf_kernel_needs_a_chunk(ggml_type):
+    """The GEMV over rows of any length clamps its loads to a row's last chunk: a row of no values is not its."""
+    from qlin import _lib
+    f = _lib.load()["_ZN4qlin24gguf_gemv_rows_supportedEillPKvS1_"]
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
+    row = {2: 18 * 8, 8: 34 * 8, 12: 144, 13: 176, 14: 210, 20: 18 * 8, 23: 136}[ggml_type]  # bytes of 256 values
+    assert not f(ggml_type, 0, 0, 4096, 4096)
+    assert f(ggml_type, 256, row, 4096, 4096) and f(ggml_type, 16384, 64 * row, 4096, 4096)
+    assert not f(ggml_type, 16384 + 256, 65 * row, 4096, 4096)
