@@ -8,7 +8,7 @@
 //   bwd_rows_kernel: a[m, n] = fp16((dy[m, n] s[n]) 2^-E[m]), E[m] the exponent of the row's
 //     max |dy s| (one rounding, no overflow or underflow of the row's large values), rows
 //     zero-padded to a multiple of 128;
-//   bwd_gemm_kernel: c = a q over n with fp16 MFMA (the int8 codes are exact fp16), one
+//   bwd_gemm_kernel, bwd_gemm_pair_kernel: c = a q over n with fp16 MFMA (the int8 codes are exact fp16), one
 //     workgroup per 128 rows x 256 columns of dx; the weight tile goes to LDS as stored (rows
 //     of n, k contiguous) and each MFMA fragment (8 consecutive n of one column) is one
 //     transposing 8-byte LDS read, widened in registers; the epilogue scales rows by 2^E[m],
@@ -128,6 +128,54 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(uint32_t w0, uint32_t w1) {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
 
+// The output of a tile, four passes of 32 rows through LDS (the pipeline buffers are no longer read; the caller has
+// synchronized): element (row, c) at row * BW_OW + c + 4 (c / 16).
+template <int G>
+__device__ __forceinline__ void bwd_store(const BwdGemmArgs& p, const f32x16 (&acc)[2][2], uint8_t* smem, int64_t m0, int64_t k0,
+                                          int tid) {
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r32 = lane & 31, h = lane >> 5, wm = wave >> 2, wk = wave & 3;
+    float* ot = reinterpret_cast<float*>(smem);
+    const bool vec = (p.ldo % 8 == 0) && ((uintptr_t)p.out % 16 == 0);
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {  // unrolled: acc[pass % 2] must stay in registers
+        if (pass) __syncthreads();
+        // C layout: lane l, register e holds row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32
+        if (wm == pass / 2) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int row = 8 * (e / 4) + 4 * h + e % 4, c = 64 * wk + 32 * j + r32;
+                    ot[row * BW_OW + c + 4 * (c >> 4)] = acc[pass % 2][j][e];
+                }
+        }
+        __syncthreads();
+        const int row = 4 * wave + (lane >> 4), run = lane & 15;
+        const float* src = ot + row * BW_OW + 20 * run;
+        float v[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 t = *reinterpret_cast<const f32x4*>(src + 4 * q);
+            v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
+        }
+        const int64_t m = m0 + 32 * pass + row, k = k0 + 16 * run;
+        const int E = p.e[min(m, p.M - 1)];
+        if constexpr (G > 0) {
+            hadamard16<G>(v, lane);
+            const float nrm = hadamard_norm<G>();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[i] *= nrm;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = __builtin_ldexpf(v[i], E);
+        if (m < p.M && k < p.K) {
+            store8_rt(p.out, p.out_dt, m * p.ldo + k, v, 8, vec);
+            store8_rt(p.out, p.out_dt, m * p.ldo + k + 8, v + 8, 8, vec);
+        }
+    }
+}
+
 // dx tile: rows m0 .. m0 + 127, columns k0 .. k0 + 255.  Wave w = 4 wm + wk owns rows 64 wm .. + 63 and
 // columns 64 wk .. + 63 of the tile (2 x 2 sub-tiles of 32 x 32).  A stage is 64 values of n: a tile
 // [128][64] fp16 and weight tile [64][256] int8, both brought in by LDS DMA as they lie in memory; the
@@ -142,8 +190,8 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 //   2t - 1; their buffers are refilled from phase 2t + 2 and 2t on: in stage t + 1 and stage t;
 //   a wave's requests of stage t - 2 (a tile t + 1, weight tile t + 2) have landed before the barrier that
 //   ends its memory phase t: 8 younger ones may be outstanding.  Their first reads are in phase 2t + 2.
-// Against the same tile through registers with all waves in phase (matrix cores about a third busy), M1056
-// K6144 N16384: 311 -> 214 us, 992 TFLOP/s; 216 of 256 CUs have a tile there and 8% of the tile rows are padding.
+// Against the same tile through registers with all waves in phase (bwd_gemm_pair_kernel below; matrix cores about a
+// third busy), M1056 K6144 N16384: 311 -> 214 us, 992 TFLOP/s; 216 of 256 CUs have a tile there and 8% of the tile rows are padding.
 template <int G>
 __global__ __launch_bounds__(512) void bwd_gemm_kernel(BwdGemmArgs p) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[4 * BW_BUF];
@@ -291,47 +339,100 @@ __global__ __launch_bounds__(512) void bwd_gemm_kernel(BwdGemmArgs p) {
     if (!wm) barrier();
     wait_vmcnt<0>();
     __syncthreads();  // every wave is past the main loop, its DMAs included
-    // epilogue, four passes of 32 rows through LDS (the pipeline buffers are no longer read):
-    // element (row, c) at row * BW_OW + c + 4 (c / 16)
-    float* ot = reinterpret_cast<float*>(smem);
-    const bool vec = (p.ldo % 8 == 0) && ((uintptr_t)p.out % 16 == 0);
+    bwd_store<G>(p, acc, smem, m0, k0, tid);
+}
+
+struct BwdRegs {
+    u32x4 a[2];  // 16 halves of one row of the a tile
+    u32x4 b[2];  // 16 int8 of each of two weight rows
+};
+
+// The same tile and fragments with all waves in phase, for short sums, mostly on grids of more than one round (run_bwd_gemm):
+// through registers into two LDS buffers of 34 KiB, and at most 128 registers (a few spilled), so that two workgroups
+// share a CU and one's start and output overlap the other's sum.  A stage's loads are issued two stages before it is
+// computed; loads past the last stage re-read it and are never computed.  A tile LDS row has 8 halves of padding.
+template <int G>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) void bwd_gemm_pair_kernel(BwdGemmArgs p) {
+    constexpr int LS = BW_BN + 8, ASZ = BW_BM * LS * 2, BUF = ASZ + BW_BN * BW_BK;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * BUF];
+    static_assert(32 * BW_OW * 4 <= 2 * BUF, "output staging must fit");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r32 = lane & 31, h = lane >> 5, wm = wave >> 2, wk = wave & 3;
+    const int64_t m0 = (int64_t)blockIdx.y * BW_BM, k0 = (int64_t)blockIdx.x * BW_BK;
+    // global load assignment: a row tid / 4, 16 halves at 16 (tid % 4); weight rows tid / 16 and 32 + tid / 16 of the
+    // stage, 16 bytes at column 16 (tid % 16) of the tile
+    const f16* ap = p.a + min(m0 + tid / 4, p.M - 1) * p.lda + 16 * (tid & 3);
+    const int brow = tid >> 4, bc = tid & 15;
+    const int8_t* bp = p.b + min(k0 + 16 * bc, p.K - 16);  // columns past K re-read (never stored)
+    const int last = (int)(p.lda / BW_BN) - 1;             // an odd number: lda is N rounded up to 128
+    auto load = [&](int s, BwdRegs& r) {
+        const u32x4* pa = reinterpret_cast<const u32x4*>(ap + (int64_t)BW_BN * s);
+        r.a[0] = pa[0];
+        r.a[1] = pa[1];
 #pragma unroll
-    for (int pass = 0; pass < 4; ++pass) {  // unrolled: acc[pass % 2] must stay in registers
-        if (pass) __syncthreads();
-        // C layout: lane l, register e holds row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32
-        if (wm == pass / 2) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int row = 8 * (e / 4) + 4 * h + e % 4, c = 64 * wk + 32 * j + r32;
-                    ot[row * BW_OW + c + 4 * (c >> 4)] = acc[pass % 2][j][e];
-                }
+        for (int i = 0; i < 2; ++i) {
+            const int64_t n = min((int64_t)BW_BN * s + 32 * i + brow, p.N - 1);  // rows past N meet a = 0
+            r.b[i] = *reinterpret_cast<const u32x4*>(bp + n * p.ldb);
         }
+    };
+    auto store = [&](const BwdRegs& r, int buf) {
+        f16* ad = reinterpret_cast<f16*>(smem + buf * BUF) + (tid >> 2) * LS + 16 * (tid & 3);
+        uint8_t* bs = smem + buf * BUF + ASZ;
+        *reinterpret_cast<u32x4*>(ad) = r.a[0];
+        *reinterpret_cast<u32x4*>(ad + 8) = r.a[1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int row = 32 * i + brow;
+            *reinterpret_cast<u32x4*>(bs + row * BW_BK + 16 * bw_chunk(row, bc)) = r.b[i];
+        }
+    };
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    const int gi = lane & 15, g = lane >> 4;  // the transposing reads of bwd_gemm_kernel
+    auto compute = [&](int buf) {
+        const f16* as = reinterpret_cast<const f16*>(smem + buf * BUF);
+        const uint8_t* bs = smem + buf * BUF + ASZ;
+#pragma unroll
+        for (int st = 0; st < BW_BN / 16; ++st) {
+            f16x8 af[2], bf[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                af[i] = *reinterpret_cast<const f16x8*>(as + (64 * wm + 32 * i + r32) * LS + 16 * st + 8 * h);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int row = 16 * st + 8 * (g >> 1) + (gi >> 1), kc = 64 * wk + 32 * j + 16 * (g & 1);
+                const uint8_t* src = bs + row * BW_BK + 16 * bw_chunk(row, kc >> 4) + 8 * (gi & 1);
+                const v2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)src);
+                bf[j] = i8x8_to_f16((uint32_t)w.x, (uint32_t)w.y);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // stage s lives in register set s % 2 and LDS buffer s % 2
+    BwdRegs r0, r1;
+    load(0, r0);
+    load(1, r1);
+    store(r0, 0);
+    __syncthreads();
+    for (int s = 0; s < last; s += 2) {
+        load(min(s + 2, last), r0);
+        compute(0);
+        store(r1, 1);
         __syncthreads();
-        const int row = 4 * wave + (lane >> 4), run = lane & 15;
-        const float* src = ot + row * BW_OW + 20 * run;
-        float v[16];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 t = *reinterpret_cast<const f32x4*>(src + 4 * q);
-            v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
-        }
-        const int64_t m = m0 + 32 * pass + row, k = k0 + 16 * run;
-        const int E = p.e[min(m, p.M - 1)];
-        if constexpr (G > 0) {
-            hadamard16<G>(v, lane);
-            const float nrm = hadamard_norm<G>();
-#pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] *= nrm;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = __builtin_ldexpf(v[i], E);
-        if (m < p.M && k < p.K) {
-            store8_rt(p.out, p.out_dt, m * p.ldo + k, v, 8, vec);
-            store8_rt(p.out, p.out_dt, m * p.ldo + k + 8, v + 8, 8, vec);
-        }
+        load(min(s + 3, last), r1);
+        compute(1);
+        store(r0, 0);
+        __syncthreads();
     }
+    bwd_store<G>(p, acc, smem, m0, k0, tid);
 }
 
 }  // namespace
@@ -360,17 +461,31 @@ hipError_t run_bwd_rows(const void* dy, int dy_dt, int64_t ldd, int64_t M, int64
     return hipGetLastError();
 }
 
+// Short sums on more than one round of the 256 CUs: the kernel that two workgroups share a CU with.  In the other
+// one's four stages of loads and its output overlap nothing, and the more rounds, the longer a sum has to be to win
+// that back.  us for gradient rows and GEMM, bf16, G 256, two-group and pair kernel:
+//   288 tiles (M2200 K4096): N512 44.2, 40.0; N1280 61.7, 61.2; N1536 67.2, 66.5; N1792 72.7, 73.1; N2048 78.3, 80.3
+//   504 tiles (M2600 K6144): N512 47.6, 43.5; N1536 76.6, 73.4; N2048 90.5, 89.2; N2304 98.7, 98.7; N2560 105.5, 106.2
+//   2016 tiles (M4600 K14336): N512 154, 123; N1024 205, 179; N2048 316, 304; N2304 344, 336; N2560 372, 368
+//   4800 tiles (M9504 K16384): N2304 792, 781; N2560 854, 869
+// and sums of two stages on any grid (M64 K4096 N128 16.4, 16.1; N256 17.7, 17.8; N512 19.8, 21.2).
+bool bwd_gemm_pair(int64_t tiles, int64_t stages) {
+    return stages <= (tiles > 512 ? 36 : tiles > 416 ? 32 : tiles > 256 ? 26 : 2);
+}
+
 hipError_t run_bwd_gemm(const BwdGemmArgs& p, hipStream_t st) {
     if (p.M == 0 || p.K == 0) return hipSuccess;
-    // the kernel's loads assume: K a multiple of 16 (4-byte weight loads from clamped columns),
+    // the kernels' loads assume: K a multiple of 16 (16-byte weight loads from clamped columns),
     // 16-byte aligned weight rows, lda a multiple of 128 covering N, N >= 1
     if (p.K % 16 || p.ldb % 16 || (uintptr_t)p.b % 16 || p.lda % (2 * BW_BN) || p.lda < p.N || p.N < 1 ||
         (uintptr_t)p.a % 16)
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)((p.K + BW_BK - 1) / BW_BK), (unsigned)((p.M + BW_BM - 1) / BW_BM));
+    const bool pair = bwd_gemm_pair((int64_t)grid.x * grid.y, p.lda / BW_BN);
     bool ok = false;
     auto go = [&]<int G>() {
-        hipLaunchKernelGGL((bwd_gemm_kernel<G>), grid, dim3(512), 0, st, p);
+        if (pair) hipLaunchKernelGGL((bwd_gemm_pair_kernel<G>), grid, dim3(512), 0, st, p);
+        else hipLaunchKernelGGL((bwd_gemm_kernel<G>), grid, dim3(512), 0, st, p);
         ok = true;
     };
     if (!dispatch_group(p.G, go) || !ok) return hipErrorInvalidValue;

@@ -429,6 +429,9 @@ struct BwdGemmArgs {
 hipError_t run_bwd_rows(const void* dy, int dy_dt, int64_t ldd, int64_t M, int64_t N, const void* s, int s_dt,
                         int64_t s_stride, f16* a, int64_t lda, int32_t* e, hipStream_t st);
 hipError_t run_bwd_gemm(const BwdGemmArgs& p, hipStream_t st);
+// Whether a gradient GEMM of so many 128 x 256 tiles and 64-value stages takes the kernel that two workgroups share a
+// CU with.
+bool bwd_gemm_pair(int64_t tiles, int64_t stages);
 // K splits of the LoRA down-projection for this shape (the workspace holds that many partials).
 constexpr int LORA_MAX_SPLITS = 32;
 int lora_splits(int64_t M, int64_t K, int64_t R);

@@ -291,3 +291,14 @@ def test_one_row_gguf_kernel_needs_a_chunk(ggml_type):
     assert not f(ggml_type, 0, 0, 4096, 4096)
     assert f(ggml_type, 256, row, 4096, 4096) and f(ggml_type, 16384, 64 * row, 4096, 4096)
     assert not f(ggml_type, 16384 + 256, 65 * row, 4096, 4096)
+
+
+def test_gradient_route_by_rounds_and_stages():
+    """Short sums on grids past one round of the CUs go to the gradient kernel that two workgroups share a CU with."""
+    from qlin import _lib
+    f = _lib.load()["_ZN4qlin13bwd_gemm_pairEll"]
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int64, ctypes.c_int64]
+    for tiles, stages in ((16, 2), (256, 2), (257, 26), (416, 26), (432, 32), (512, 32), (513, 36), (8192, 36)):
+        assert f(tiles, stages) and not f(tiles, stages + 2), (tiles, stages)
+    assert f(2048, 16)  # M4000 K16384 N1024
+    assert not f(216, 256)  # M1056 K6144 N16384

@@ -79,6 +79,14 @@ def test_grad_input(n, m, k):
     _check(dx, dy, q.float().T / 2)
 
 
+# 306, 442 and 561 tiles, rows and columns of the last ones past the matrix: the kernel that two workgroups share a CU
+# with up to 26, 32 and 36 stages of 64, and the one past them
+@pytest.mark.parametrize("m,n", [(2200, 1), (2200, 129), (2200, 300), (2200, 1664), (2200, 1665), (3300, 2048), (3300, 2049),
+                                 (4100, 2304), (4100, 2305)])
+def test_grad_input_rounds(m, n):
+    test_grad_input(n, m, 4112)
+
+
 @pytest.mark.parametrize("qtype,k", [("Q8_0", 8224), ("Q8_0", 16384), ("Q6_K", 8448), ("Q6_K", 16640)])
 def test_wide_rows_decoded(qtype, k):
     """Rows on both sides of the limits of the decode that keeps a row in registers (8192, 16384)."""
