@@ -802,10 +802,11 @@ static qlin_status gguf_linear_impl(const qlin_tensor* x, const void* weight, in
         (M <= GGUF_SMALLM_MAX_M || K % 64 || (uintptr_t)workspace % 16 ||
          gguf_decode_rows(N, K, (int64_t)workspace_bytes - (int64_t)ws_gguf(M, N, K, ggml_type)) <= 0))
         return QLIN_NOT_FUSED;
-    // one row: fp16 rows of 16, 32 or 64 chunks keep them in registers, other lengths and dtypes take
-    // the GEMV that walks them (and normalizes in the kernel)
+    // one row: fp16 rows of 16, 32 or 64 chunks keep them in registers and short ones over few weights take the
+    // 16-row kernel; other lengths and dtypes take the GEMV that walks them (and normalizes in the kernel)
     if (M == 1 && aligned && gguf_gemv_rows_supported(ggml_type, K, row_bytes, weight, X.data) &&
-        !(X.dtype == QLIN_DT_F16 && gguf_gemv_supported(ggml_type, 1, K, row_bytes, weight, X.data))) {
+        !(X.dtype == QLIN_DT_F16 &&
+          (gguf_gemv_supported(ggml_type, 1, K, row_bytes, weight, X.data) || gguf_short_row(ggml_type, N, K)))) {
         GgufGemvArgs g;
         g.type = ggml_type; g.x = X.data; g.x_dtype = X.dtype; g.w = (const uint8_t*)weight; g.row_bytes = row_bytes;
         g.N = (int)N; g.K = (int)K;

@@ -937,6 +937,18 @@ bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void
     return ok;
 }
 
+// Short fp16 rows over few weights stay with the 16-row MFMA kernel: neither launches a prologue for them, and what
+// counts is the time to the first bytes, which here waits for the operand's trip through LDS.  us, 16-row kernel and
+// GEMV: Q5_K K256 N64 2.6, 3.3, N8192 3.4, 3.8, N16384 5.2, 5.4; Q4_K K256 N4096 2.9, 3.3, N12288 4.8, 4.9, N16384 5.1,
+// 5.0; K768 N64 2.7, 3.1, N3072 3.3, 3.4, N8192 4.0, 3.7; K512 N1024 3.1, 3.15, N4096 3.5, 3.4.  Q4_0 and Q5_K also at
+// the other lengths: Q4_0 K512 N4096 3.4, 3.6; K1024 N256 3.2, 3.3, N2048 3.60, 3.65; K1536 N64 3.2, 3.3, N1024 3.7,
+// 3.65; K2304 N64 4.1, 3.5.  Q6_K and Q8_0 gain at every length (Q6_K K256 N64 19.8, 3.5; Q8_0 K256 2.8, 2.65).
+bool gguf_short_row(int type, int64_t N, int64_t K) {
+    if (K < 1 || K % 256 || K >= 2048 || type == gguf::Q6_K || type == gguf::Q8_0) return false;
+    if (K == 256 || K == 768) return N * K <= 3 << 20;
+    return (type == gguf::Q4_0 || type == gguf::Q5_K) && N * K <= 2 << 20;
+}
+
 hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st) {
     if (!gguf_gemv_rows_supported(a.type, a.K, a.row_bytes, a.w, a.x)) return hipErrorInvalidValue;
     if (a.y_dtype != DT_F32 && a.y_dtype != DT_F16 && a.y_dtype != DT_BF16) return hipErrorInvalidValue;

@@ -184,6 +184,8 @@ hipError_t run_gguf_gemv(const GgufGemvArgs& a, hipStream_t st);
 // The GEMV over rows of any whole number of chunks (64 values for Q8_0, else 128) up to 16384, at
 // least one.
 bool gguf_gemv_rows_supported(int type, int64_t K, int64_t row_bytes, const void* w, const void* x);
+// An fp16 row that the 16-row MFMA kernel takes sooner.
+bool gguf_short_row(int type, int64_t N, int64_t K);
 hipError_t run_gguf_gemv_rows(const GgufGemvArgs& a, hipStream_t st);
 
 // ---- weight-only fp16 MFMA tile GEMM (gemm_f16.hip) ----

@@ -302,3 +302,16 @@ def test_gradient_route_by_rounds_and_stages():
         assert f(tiles, stages) and not f(tiles, stages + 2), (tiles, stages)
     assert f(2048, 16)  # M4000 K16384 N1024
     assert not f(216, 256)  # M1056 K6144 N16384
+
+
+def test_short_fp16_rows_stay_with_the_16_row_kernel():
+    from qlin import _lib
+    f = _lib.load()["_ZN4qlin14gguf_short_rowEill"]
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
+    q4_0, q8_0, q4_k, q5_k, q6_k = 2, 8, 12, 13, 14
+    for t in (q4_0, q4_k, q5_k):
+        assert f(t, 12288, 256) and not f(t, 12289, 256) and f(t, 4096, 768) and not f(t, 4097, 768)
+        assert not f(t, 64, 2048) and not f(t, 64, 384) and not f(t, 64, 0)
+    assert f(q4_0, 4096, 512) and f(q5_k, 2048, 1024) and not f(q5_k, 2049, 1024) and not f(q4_k, 64, 512)
+    for t in (q6_k, q8_0):
+        assert not f(t, 64, 256)
