@@ -176,6 +176,8 @@ def test_int8_residual_fused_equals_separate(m, n, k, odt, rdt):
     (1024, 4096, 1024, 4, 64),   # grid decoded once, then the int8 DMA GEMM (128 x 256 tiles)
     (2600, 6100, 512, 6, 64),    # 264 tiles of 256 x 256: the last 40 rows on 128 x 256 tiles
     (1000, 5100, 1024, 6, 64),   # the same with 2 x 5 waves on 128 x 160 tiles (256 of them)
+    (3585, 3500, 3584, 4, 64),   # 210 tiles of 256 x 256 in the two-group loop
+    (2305, 8100, 3840, 6, 64),   # the same past a whole round: the last 257 rows on 128 x 128 tiles
     (300, 24600, 1024, 6, 64),   # one 256-row tile over a wide grid: the fused-decode GEMM
     (100, 1000, 1024, 4, 16),    # group 16: the 128 x 128 decode-in-load kernel, residual kernel after
     (8, 512, 1024, 6, 64),       # small M

@@ -292,8 +292,24 @@ def test_w4a8_lora_fused_into_gemm(bits, m, n, r, fdt, fused_calls):
     """A8 calls whose weight grid is decoded once (from 512 rows, and above 32 rows on grids of fewer
     than 192 tiles of 256 x 256), then the DMA GEMM that carries the LoRA term, at each of its tile
     shapes: 256 x 256 from 192 such tiles, else 128 x 256, 128 x 128 or 128 x 64."""
+    _w4a8_lora_fused(bits, m, n, 1024, r, fdt, fused_calls)
+
+
+@pytest.mark.parametrize("m,n", [(3585, 3500), (600, 16400)])  # 210 and 195 tiles of 256 x 256, the last ones ragged
+@pytest.mark.parametrize("bits,k,r,fdt", [
+    (4, 3584, 8, torch.bfloat16), (6, 3712, 48, torch.bfloat16), (4, 3712, 64, torch.bfloat16),
+    (4, 3584, 128, torch.bfloat16),  # ranks above 64 (fp32 factors: 32) in two passes
+    (6, 3584, 8, torch.float16), (4, 3712, 48, torch.float16), (4, 3584, 64, torch.float16), (6, 3584, 128, torch.float16),
+    (6, 3584, 32, torch.float32), (4, 3712, 64, torch.float32),
+])
+def test_w4a8_lora_fused_into_two_group_gemm(bits, k, r, fdt, m, n, fused_calls):
+    """Rows of 3584 values and more: 256 x 256 tiles whose accumulators are 16 x 16 sub-tiles."""
+    _w4a8_lora_fused(bits, m, n, k, r, fdt, fused_calls)
+
+
+def _w4a8_lora_fused(bits, m, n, k, r, fdt, fused_calls):
     Q = qlin()
-    k, g, gs = 1024, 256, 64
+    g, gs = (256, 64) if k % 256 == 0 else (128, 64)
     gen = torch.Generator().manual_seed(30 + bits)
     hi = 15 if bits == 4 else 63
     codes = torch.randint(1, hi + 1, (n, k), generator=gen, dtype=torch.int32)
