@@ -24,9 +24,11 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // KIND 0: v_mfma_f32_32x32x16_f16, 1: v_mfma_f32_16x16x32_f16, 2: v_mfma_i32_32x32x32_i8,
-// 3: v_mfma_i32_16x16x64_i8.
+// 3: v_mfma_i32_16x16x64_i8.  The 16 x 16 loops are compiled for 512 threads (and launched with 256): with the registers
+// of 256 the compiler moves the accumulators through accumulation registers every round, 52 moves for 8 MFMAs, and
+// those are what is measured.
 template <int KIND>
-__global__ __launch_bounds__(256) void mfma_rate_kernel(float* out, int iters) {
+__global__ __launch_bounds__(KIND % 2 ? 512 : 256) void mfma_rate_kernel(float* out, int iters) {
     const int t = threadIdx.x;
     f16x8 a, b;
 #pragma unroll
