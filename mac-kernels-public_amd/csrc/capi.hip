@@ -192,7 +192,7 @@ size_t ws_gguf(int64_t M, int64_t N, int64_t K, int type) {
 // holds at least one chunk of GGUF_DECODE_CHUNK_ROWS rows (or all N); the size query asks for
 // min(N, the rows of GGUF_DECODE_BYTES_MAX) rows.
 constexpr int64_t GGUF_DECODE_BYTES_MAX = 256ll << 20;
-constexpr int64_t GGUF_DECODE_CHUNK_ROWS = 128;  // the GEMM's tile height along N
+constexpr int64_t GGUF_DECODE_CHUNK_ROWS = 128;  // the ring kernel's tile height along N, half of the 256 x 256 tiles'
 // Rows of one decoded chunk that `bytes` of workspace hold (a multiple of the chunk unit, or N),
 // 0 when not even one unit fits.
 int64_t gguf_decode_rows(int64_t N, int64_t K, int64_t bytes) {

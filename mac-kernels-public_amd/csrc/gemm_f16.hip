@@ -1147,7 +1147,7 @@ hipError_t launch1(const GemmF16Args& a, hipStream_t st) {
         if (vec && tiles(256, 256) >= 160) {
             const dim3 grid((unsigned)tiles(256, 256));
             const int64_t m1 = a.lora.t ? 0 : tail_split_rows(a.M, a.N);
-            if (m1) {  // whole rounds of 256 x 256 tiles, then the rest as one round of 128 x 256 tiles
+            if (m1) {  // whole rounds of 256 x 256 tiles, then the rest as one round of smaller ones
                 GemmF16Args top = a, rest = a;
                 top.M = m1;
                 rest.M = a.M - m1;

@@ -1041,9 +1041,9 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_i8dma_kernel(GemmI8Args p
 }
 
 // 256 x 256 tiles over the decoded int8 grid: the main loop of gemm_pp.h, then the epilogue of
-// gemm_i8dma_kernel, in passes of 64 rows.  Against the 32 x 32 loop with one
-// barrier a k-tile that it replaces: W6A8 MLP 5120 -> 13824 -> 5120 at 9504 rows, both calls whole, 1542 -> 1412 us;
-// W4A8 M4096 K3072 N12288 190 us with either (24 k-tiles: prologue and epilogue weigh more).
+// gemm_i8dma_kernel, in passes of 64 rows.  Against that kernel's 32 x 32 loop with one barrier a k-tile: W6A8 MLP
+// 5120 -> 13824 -> 5120 at 9504 rows, both calls whole, 1542 -> 1412 us.  Rows shorter than 3584 values stay with that
+// kernel (launch_o).
 template <int LDU = -1>
 __global__ __launch_bounds__(512) void gemm_i8pp_kernel(GemmI8Args p, const int8_t* __restrict__ w8) {
     constexpr int NT = 512, BT = 256;
@@ -1332,7 +1332,7 @@ hipError_t launch_o(const GemmI8Args& p, hipStream_t st) {
         // N8192 157, 153; M2500 K5120 N13824 241, 219; M1500 K16384 N8192 259, 222)
         const bool pp = p.K >= 3584;
         const int64_t m1 = ldu == -1 && tiles(256, 256) >= 192 ? tail_split_rows(p.M, p.N) : 0;
-        if (m1) {  // whole rounds of 256 x 256 tiles, then the rest as one round of 128 x 256 tiles
+        if (m1) {  // whole rounds of 256 x 256 tiles, then the rest as one round of 128-row tiles
             GemmI8Args top = p, rest = p;
             top.M = m1;
             rest.M = p.M - m1;

@@ -1,4 +1,4 @@
-// Main loop of the 256 x 256 tile GEMMs: two groups of four waves take turns on the matrix cores.
+// Main loops of the 256 x 256 tile GEMMs: two groups of four waves take turns on the matrix cores.
 //
 // A k-tile is 128 bytes of every activation row (64 fp16 or 128 int8 values).  Wave w = 4 wm + wn owns
 // rows 128 wm .. and columns 64 wn .. of the tile (8 x 4 sub-tiles of 16 x 16) and works through a
@@ -19,13 +19,14 @@
 // of it.  Both groups have read a half-tile, and waited for the reads, at least one barrier before any
 // wave's request overwrites it.
 //
-// What bounds it: the loop keeps the matrix cores 95% busy (2160 of 2048 cycles a k-tile) and the card
+// What bounds it: the loop keeps the matrix cores 95% busy (2048 of 2160 cycles a k-tile) and the card
 // then lowers its clock to 1.5 - 1.6 GHz, so power decides.  16 x 16 sub-tiles draw less than 32 x 32
 // (fragments held, no DMA: 1.95 against 1.66 GHz): 8192 x 8192 x 4096 fp16 1431 against 1253 TFLOP/s.
 // DMAs issued between the MFMAs instead of in the memory phase: 1385; ahead of the fragment reads, with
-// 32 x 32 sub-tiles: 1092 against 1253 (the reads then wait behind them).  int8 weights widened to fp16
-// here (40 VALU operations a step, in either phase) took 3082 - 3448 cycles a k-tile, 1206 - 1262
-// TFLOP/s: the callers hand over fp16.
+// 32 x 32 sub-tiles: 1092 against 1253 (the reads then wait behind them).  PingPong takes both operands as
+// the MFMAs do.  int8 weights against fp16 activations have a loop of their own, PingPongW8 below: widened
+// between these MFMAs of 16 cycles (40 VALU operations a step, in either phase) they took 3082 - 3448 cycles a
+// k-tile, 1206 - 1262 TFLOP/s.
 #pragma once
 #include <type_traits>
 

@@ -902,8 +902,9 @@ hipError_t launch_rows_nt(const GgufGemvArgs& a, hipStream_t st) {
 
 // Workgroups of 8 waves (twice the loads in flight per operand) for large Q4_K tensors: K5120 N13824 14.3
 // -> 13.0 us, K13824 N5120 16.4 -> 15.2, K4096 N14336 11.7 -> 11.2, K16384 N8192 21.5 -> 20.4; below 50
-// million weights the longer start loses (K5120 N8192 8.6 against 10.0), and the other types are
-// limited by their decode (Q5_K K3584 N18944 16.9 against 17.3, Q6_K K13824 N5120 19.9 against 21.1).
+// million weights the longer start loses (K5120 N8192 8.6 against 10.0).  Q5_K goes either way there (K4096 N14336
+// 14.0 -> 13.3, K16384 N8192 25.3 -> 24.5, but K8192 N16384 24.5 -> 24.8, K3584 N18944 16.9 -> 17.3, K13824 N5120 18.7
+// -> 19.6), Q6_K lost where it was measured (K13824 N5120 19.9 -> 21.1); both and the types not measured keep 4 waves.
 template <int T, typename TX>
 hipError_t launch_rows(const GgufGemvArgs& a, hipStream_t st) {
     if constexpr (T == gguf::Q4_K) {
